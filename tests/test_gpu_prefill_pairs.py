@@ -1,0 +1,58 @@
+"""The balanced prefill's wave-pair kernel (head_dim 256: 192-row units, 32-key tiles, a score wave
+one step ahead of its output wave, tiles loaded two steps ahead) at the edges of its pipeline: runs
+of one, two and three tiles, units of one tile behind each other, chunks and contexts just below, at
+and above a tile, wave pairs without rows or without a visible key, groups that give a workgroup 192,
+16 or 3 tokens, and page ids outside the cache, all against the oracle within the repository's
+prefill tolerance (P and the output are rounded to 16 bits, as in the oracle)."""
+import pytest
+import torch
+
+from helpers import ATOL, RTOL, bits, say
+from oracle.ref_torch import ref_gqa_prefill_paged
+from tileinfer_amd.kernels.gqa_prefill_paged import gqa_prefill_paged_fn
+from tileinfer_amd.workloads import prefill_step
+
+pytestmark = pytest.mark.gpu
+
+
+def both(step, dev, causal=True):
+    out = gqa_prefill_paged_fn(step.q.to(dev), step.k_cache.to(dev), step.v_cache.to(dev),
+                               step.block_table.to(dev), step.cu_seqlens_q.to(dev),
+                               step.seqlen_k.to(dev), step.max_seqlen_q, step.page_size,
+                               causal=causal, schedule="balanced")
+    ref = ref_gqa_prefill_paged(step.q, step.k_cache, step.v_cache, step.block_table,
+                                step.cu_seqlens_q, step.seqlen_k, step.page_size, causal)
+    return out, ref
+
+
+@pytest.mark.parametrize("hq,hkv", [(24, 4), (2, 2), (12, 1), (64, 1)])
+@pytest.mark.parametrize("q_lens,kv_lens", [
+    ([1], [1]), ([31], [31]), ([32], [32]), ([33], [33]), ([1], [65]), ([32, 33], [96, 64]),
+    ([1] * 70, [1] * 70),                        # one-tile units behind each other
+    ([3, 1, 40, 0, 5], [3, 33, 129, 7, 0]),      # an empty chunk, a chunk without context
+    ([200], [231]), ([64, 1, 1], [64, 900, 32]),
+])
+def test_pipeline_edges_vs_oracle(q_lens, kv_lens, hq, hkv, dev):
+    say(f"prefill pairs q={q_lens} kv={kv_lens} heads={hq}/{hkv}")
+    step = prefill_step(q_lens, kv_lens, seed=51, hq=hq, hkv=hkv)
+    for causal in (True, False):
+        out, ref = both(step, dev, causal)
+        torch.testing.assert_close(out.float().cpu(), ref.float(), atol=ATOL, rtol=RTOL)
+
+
+def test_values_outside_every_mask_stay_out(dev):
+    """Non-finite K and V at positions that no query of the call may see leave the output as it is:
+    tokens behind the context in its last page, and tokens that only later query blocks see."""
+    step = prefill_step([400], [470], seed=52)
+    clean, _ = both(step, dev)
+    for first in (470, 448):  # past the context; the last tile, seen by tokens 378.. of the chunk
+        kc, vc = step.k_cache.clone(), step.v_cache.clone()
+        for pos in range(first, 480 if first == 470 else 470):
+            page, row = int(step.block_table[0, pos // 16]), pos % 16
+            kc[page, row] = float("nan")
+            vc[page, row] = float("inf")
+        out = gqa_prefill_paged_fn(step.q.to(dev), kc.to(dev), vc.to(dev), step.block_table.to(dev),
+                                   step.cu_seqlens_q.to(dev), step.seqlen_k.to(dev), 400, 16,
+                                   schedule="balanced")
+        keep = 400 if first == 470 else 352  # whole query blocks of 32 tokens before position 448
+        assert torch.equal(bits(out[:keep]), bits(clean[:keep])), first

@@ -84,10 +84,12 @@ typedef __attribute__((address_space(3))) void* lds_ptr_t;
 // loads only add to what a count waits for), and the kernel waits for these loads explicitly
 // before each stage barrier. The builtin form instead makes the compiler wait for every load
 // into a stage array before reading that array, all loads issued since included, which defeats
-// a pipeline that keeps two tiles in flight.
+// a pipeline that keeps two tiles in flight. Nor does the compiler's hazard recogniser see it: a
+// descriptor word written by v_readfirstlane or v_readlane (VALU) must be five wait states old when
+// a buffer instruction reads it, and m0 one, which the s_nop provides.
 __device__ __forceinline__ void load_lds16(u32x4 rsrc, uint32_t voff, const uint16_t* lds) {
   const uint32_t m0 = uint32_t(reinterpret_cast<uintptr_t>((lds_ptr_t)(lds)));
-  asm volatile("buffer_load_dwordx4 %0, %1, 0 offen lds" ::"v"(voff), "s"(rsrc), "{m0}"(m0)
+  asm volatile("s_nop 4\n\tbuffer_load_dwordx4 %0, %1, 0 offen lds" ::"v"(voff), "s"(rsrc), "{m0}"(m0)
                : "memory");
 }
 
@@ -125,6 +127,19 @@ __device__ __forceinline__ int lds_swizzle(int r) { return (r ^ ((r << 1) & 8)) 
 // bytes of a row, so XOR-ing the chunk index with 2r puts every row's 32 bytes on distinct banks.
 __device__ __forceinline__ int lds_swizzle_v(int r) { return (2 * r) & 14; }
 
+// Maxima without the quieting of NaN operands that fmaxf's other spellings cost (v_max returns the
+// other operand for a quiet NaN, as fmaxf does).
+__device__ __forceinline__ float max2(float x, float y) {
+  float r;
+  asm("v_max_f32 %0, %1, %2" : "=v"(r) : "v"(x), "v"(y));
+  return r;
+}
+__device__ __forceinline__ float max3(float x, float y, float z) {
+  float r;
+  asm("v_max3_f32 %0, %1, %2, %3" : "=v"(r) : "v"(x), "v"(y), "v"(z));
+  return r;
+}
+
 // Max over the four 16-lane rows of the wave (lanes n, n+16, n+32, n+48).
 __device__ __forceinline__ float row_group_max(float x) {
   auto a = __builtin_amdgcn_permlane32_swap(__float_as_uint(x), __float_as_uint(x), false, false);
@@ -145,15 +160,17 @@ struct SeqExtent {
   int offset;  // query i sits at absolute position offset + i
 };
 
-__device__ __forceinline__ SeqExtent seq_extent(const PrefillArgs& a, int b) {
+__device__ __forceinline__ SeqExtent clamp_extent(const PrefillArgs& a, int q0, int q1, int kv) {
   SeqExtent s;
-  s.q_start = min(max(a.cu_q[b], 0), a.total_q);
-  s.q_len = min(max(a.cu_q[b + 1], s.q_start), a.total_q) - s.q_start;
-  const int kv = a.seqlen_k[b];
+  s.q_start = min(max(q0, 0), a.total_q);
+  s.q_len = min(max(q1, s.q_start), a.total_q) - s.q_start;
   const int cap = a.max_blocks * a.page_size;
   s.kv_len = kv < 0 ? 0 : (kv > cap ? cap : kv);
   s.offset = s.kv_len - s.q_len;
   return s;
+}
+__device__ __forceinline__ SeqExtent seq_extent(const PrefillArgs& a, int b) {
+  return clamp_extent(a, a.cu_q[b], a.cu_q[b + 1], a.seqlen_k[b]);
 }
 
 // Keys the query block starting at qb0 can see: j < kv_len, and j < offset + qb0 + tq under the
@@ -311,6 +328,144 @@ __global__ __launch_bounds__(kPlanThreads) void prefill_plan_kernel(PrefillArgs 
   }
 }
 
+// Runs are dealt to the XCDs in contiguous blocks: workgroup ids go round-robin over the 8 XCDs, so run i = (id % 8) * (G / 8) + id / 8 keeps consecutive runs (one KV head, query blocks
+// of one sequence, the same K/V pages) in one XCD's L2.
+__device__ __forceinline__ int run_index(const PrefillArgs& a) {
+  const int nwg = a.balanced_wgs;
+  return (nwg % kXcds == 0) ? int(blockIdx.x % kXcds) * (nwg / kXcds) + int(blockIdx.x / kXcds)
+                            : int(blockIdx.x);
+}
+
+// Uniform value of a wave.
+__device__ __forceinline__ int uni(int x) { return __builtin_amdgcn_readfirstlane(x); }
+
+// A walk over the pieces of a workgroup's run. Every wave walks the tiles it computes, and the score
+// waves a second time the tiles to be loaded. The walk's state is private to the wave and kept in
+// LDS: it is needed once per piece and would otherwise hold ~40 scalar registers through the tile
+// loop.
+// A run that starts inside a unit defers that first piece (the unit's tail) to its end:
+// every run then starts at key 0 of a unit, and the deferred tail begins about where the run's
+// last piece (the next unit's head, same cut) ended, so an XCD's workgroups sweep the keys
+// together and share pages in L2. Partial slot 0 stays the run's first piece, slot 1 its last.
+struct Walk {
+  // The current piece: key tiles [t0, t1) of unit (sequence b, KV head kvh, first row qr0), and the
+  // sequence's extent.
+  int b, kvh, qr0, t0, t1;
+  int q_start, q_len, kv_len;
+  int whole;  // all key tiles of the unit
+  int slot0;  // a cut unit's partial goes to the workgroup's slot 0 (its first piece), else 1
+  int fin;    // no piece follows
+  int pos, end, n_pairs, unit_work;  // the run's work [pos, end); the plan's pairs and their work
+  // Where the walk goes on.
+  int next_p, next_kvh, d_p, d_kvh;
+  int first, deferred, replay;
+};
+
+// Moves a walk that is not finished to its next piece; false when it has none (a run may end inside
+// a unit's fixed part). A pair's four table entries and a sequence's three lengths are each read by
+// one load, an entry per lane: read one by one, each waited for, they cost a short unit more than
+// its attention (24 prompts of 17 to 700 tokens: 139 -> 130 us per balanced call).
+__device__ __forceinline__ bool walk_next(const PrefillArgs& a, Walk& w) {
+  const int lane = threadIdx.x & 63;
+  const int pos = uni(w.pos), end = uni(w.end);
+  const int n_pairs = uni(w.n_pairs), unit_work = uni(w.unit_work);
+  int p = uni(w.next_p), kvh = uni(w.next_kvh), d_p = uni(w.d_p), d_kvh = uni(w.d_kvh);
+  bool first = uni(w.first) != 0, deferred = uni(w.deferred) != 0, replay = uni(w.replay) != 0;
+  for (;;) {
+    const PlanView v = plan_view(a);
+    const int x = v.pair_b[int64_t(lane & 3) * a.max_pairs + p];  // sequence, block, tiles, prefix
+    const int nt = __builtin_amdgcn_readlane(x, 2);
+    // The unit's key tiles occupy work [k_pos, k_pos + nt).
+    const int k_pos = kvh * unit_work + __builtin_amdgcn_readlane(x, 3) + kUnitCost;
+    const int t0 = max(pos - k_pos, 0);
+    const int t1 = min(end - k_pos, nt);
+    const bool last = k_pos + nt >= end;
+    const bool slot0 = first || replay;
+    bool go = t0 < t1;  // units without keys get their zero rows from the merge
+    if (go && first && t0 > 0 && !last) {
+      d_p = p;
+      d_kvh = kvh;
+      deferred = true;
+      first = false;
+      go = false;
+    }
+    if (go) {
+      const int b = __builtin_amdgcn_readlane(x, 0);
+      const int32_t* at = (lane & 3) < 2 ? a.cu_q + b + (lane & 1) : a.seqlen_k + b;
+      const int y = *at;
+      w.b = b;
+      w.qr0 = __builtin_amdgcn_readlane(x, 1) * a.tq * a.group;
+      w.kvh = kvh;
+      w.t0 = t0;
+      w.t1 = t1;
+      w.whole = t0 == 0 && t1 == nt;
+      w.slot0 = slot0;
+      const SeqExtent s = clamp_extent(a, __builtin_amdgcn_readlane(y, 0),
+                                       __builtin_amdgcn_readlane(y, 1),
+                                       __builtin_amdgcn_readlane(y, 2));
+      w.q_start = s.q_start;
+      w.q_len = s.q_len;
+      w.kv_len = s.kv_len;
+      first = false;
+    }
+    bool done = last || replay;
+    if (!done && ++p == n_pairs) {
+      p = 0;
+      done = ++kvh == a.hkv;
+    }
+    const bool fin = done && (!deferred || replay);
+    if (done && !fin) {
+      p = d_p;
+      kvh = d_kvh;
+      replay = true;
+    }
+    if (go || fin) {
+      w.next_p = p;
+      w.next_kvh = kvh;
+      w.d_p = d_p;
+      w.d_kvh = d_kvh;
+      w.first = first;
+      w.deferred = deferred;
+      w.replay = replay;
+      w.fin = fin;
+      return go;
+    }
+  }
+}
+
+// Starts a walk at its first piece; false when the workgroup has none.
+__device__ __forceinline__ bool walk_start(const PrefillArgs& a, Walk& w) {
+  const PlanView v = plan_view(a);
+  const int i = run_index(a);
+  const int lane = threadIdx.x & 63;
+  const int hdr = v.hdr[lane & 3];  // pairs, work per KV head, runs, total work
+  const int at = (lane & 1) ? v.wg_kvh[i] : v.wg_p[i];
+  const int p = __builtin_amdgcn_readlane(at, 0);
+  if (p < 0) return false;  // no work left for this workgroup
+  const int64_t runs = __builtin_amdgcn_readlane(hdr, 2);
+  const int64_t total = __builtin_amdgcn_readlane(hdr, 3);
+  w.n_pairs = __builtin_amdgcn_readlane(hdr, 0);
+  w.unit_work = __builtin_amdgcn_readlane(hdr, 1);
+  w.pos = int(int64_t(i) * total / runs);
+  w.end = int(int64_t(i + 1) * total / runs);
+  w.next_p = p;
+  w.next_kvh = __builtin_amdgcn_readlane(at, 1);
+  w.d_p = w.d_kvh = 0;
+  w.first = 1;
+  w.deferred = w.replay = 0;
+  return walk_next(a, w);
+}
+
+// The extent of a walk's current sequence.
+__device__ __forceinline__ SeqExtent walk_extent(const Walk& w) {
+  SeqExtent s;
+  s.q_start = uni(w.q_start);
+  s.q_len = uni(w.q_len);
+  s.kv_len = uni(w.kv_len);
+  s.offset = s.kv_len - s.q_len;
+  return s;
+}
+
 // A workgroup's rows are the (token, query head) pairs of one KV head's group, row = token * group
 // + head-in-group, 16 * C * W rows over W waves (C column tiles of 16 rows per wave). Every staged
 // K/V tile is thus shared by all query heads of the group, and every K/V operand read from LDS feeds
@@ -326,7 +481,7 @@ __global__ __launch_bounds__(kPlanThreads) void prefill_plan_kernel(PrefillArgs 
 // SMALL: pages of 4 or 8 tokens (P2 as well). A 16-key sub-tile then spans 16 / page_size pages:
 // each 1 KiB load (2 or 4 rows) lies in one page and gets that page's descriptor, and the keys
 // present in a stage are a bit mask (an absent page can share a sub-tile with a present one).
-template <int D, int C, int W, int NS, bool P2, bool SMALL, typename Tag>
+template <int D, int C, int W, int NS, bool BAL, bool P2, bool SMALL, typename Tag>
 __global__ __launch_bounds__(64 * W) void prefill_mfma_kernel(PrefillArgs a) {
   constexpr int kKT = 16 * NS;
   constexpr int KK = D / 32;
@@ -341,13 +496,6 @@ __global__ __launch_bounds__(64 * W) void prefill_mfma_kernel(PrefillArgs a) {
   constexpr int LW = 4;
   constexpr int LPW = kKT / RPB / LW;     // 1 KiB loads per loading wave per tile, each of K and V
   constexpr int ROWS = 16 * C * W;        // rows of the workgroup
-  // Register-lean forms for shapes above 8 waves (3 waves per SIMD leave 168 VGPRs): V offsets
-  // computed per read, K operands read through a ring, load offsets recomputed per tile. Each
-  // costs the 8-wave shape 1-3 % (same-process A/B), which therefore keeps the plain forms.
-  constexpr bool kLean = W > 8;
-  // K/V loads into LDS as assembly (load_lds16) or through the compiler's builtin: the 8-wave
-  // shape gains 3-6 % from the former, the 12-wave one loses ~3 % (same-process A/Bs).
-  constexpr bool kAsmLoads = !kLean;
   static_assert(W >= LW && LPW * RPB * LW == kKT && 16 % (kKT / LW) == 0,
                 "each wave's loads must lie inside one sub-tile");
 
@@ -373,23 +521,15 @@ __global__ __launch_bounds__(64 * W) void prefill_mfma_kernel(PrefillArgs a) {
   // of the A operand (keys 4g + i of sub-tile h, matching P). voff[h][dt % 8] is the element
   // offset inside a stage of d-tile dt's piece; d-tiles dt and dt + 8 differ by 128 elements
   // (the swizzle only permutes chunks inside each group of 16).
-  // Lean form: the swizzle XORs the 16-byte chunk index 2 dl + ((s % 4) / 2) with the even
-  // 2r & 14, i.e. element offset 16 (dl ^ (r & 7)) + 8 ((s % 4) / 2), so voff[h][dl] =
-  // vbase[h] + (16 dl ^ vxor[h]): one v_xad per read instead of 16 live offsets.
-  int voff[2][kLean ? 1 : 8];
-  int vbase[2], vxor[2];
+  int voff[2][8];
 #pragma unroll
   for (int hh = 0; hh < 2; ++hh) {
     const int r = 16 * hh + 4 * g + (n >> 2);
-    vbase[hh] = r * D + ((n & 3) >> 1) * 8 + (n & 1) * 4;
-    vxor[hh] = 16 * (r & 7);
-    if constexpr (!kLean) {
-      const int sw = lds_swizzle_v(r);
+    const int sw = lds_swizzle_v(r);
 #pragma unroll
-      for (int dl = 0; dl < 8; ++dl) {
-        const int y = 2 * dl + ((n & 3) >> 1);
-        voff[hh][dl] = r * D + ((y ^ sw) * 8) + (n & 1) * 4;
-      }
+    for (int dl = 0; dl < 8; ++dl) {
+      const int y = 2 * dl + ((n & 3) >> 1);
+      voff[hh][dl] = r * D + ((y ^ sw) * 8) + (n & 1) * 4;
     }
   }
   const uint32_t row_bytes = uint32_t(a.row_stride) * 2u;
@@ -518,15 +658,8 @@ __global__ __launch_bounds__(64 * W) void prefill_mfma_kernel(PrefillArgs a) {
         const uint32_t ri = uint32_t(RPB * i) * row_bytes - uint32_t(pj * ps) * row_bytes;
         const uint32_t off_k = ((lane_k ^ uint32_t(16 * lds_swizzle(RPB * i))) + lane_hi) + ri;
         const uint32_t off_v = ((lane_v ^ uint32_t(16 * lds_swizzle_v(RPB * i))) + lane_hi) + ri;
-        if constexpr (kAsmLoads) {
-          load_lds16(rsrc_words(at_bytes(a.k_cache, off), nbytes), off_k, sk + blk * 512);
-          load_lds16(rsrc_words(at_bytes(a.v_cache, off), nbytes), off_v, sv + blk * 512);
-        } else {
-          __builtin_amdgcn_raw_ptr_buffer_load_lds(make_rsrc(at_bytes(a.k_cache, off), nbytes),
-                                                   (lds_ptr_t)(sk + blk * 512), 16, off_k, 0, 0, 0);
-          __builtin_amdgcn_raw_ptr_buffer_load_lds(make_rsrc(at_bytes(a.v_cache, off), nbytes),
-                                                   (lds_ptr_t)(sv + blk * 512), 16, off_v, 0, 0, 0);
-        }
+        load_lds16(rsrc_words(at_bytes(a.k_cache, off), nbytes), off_k, sk + blk * 512);
+        load_lds16(rsrc_words(at_bytes(a.v_cache, off), nbytes), off_v, sv + blk * 512);
       }
       return;
     }
@@ -553,11 +686,6 @@ __global__ __launch_bounds__(64 * W) void prefill_mfma_kernel(PrefillArgs a) {
     const uint64_t off = uint64_t(uint32_t(bid)) * page_bytes +
                          (in_page * row_bytes + uint32_t(kvh) * uint32_t(D * 2));
     const uint32_t nbytes = rows > 0 ? uint32_t(rows - 1) * row_bytes + D * 2 : 0u;
-    // Lean form: the per-lane offsets are recomputed at every fetch (an opaque copy of the lane
-    // index keeps the compiler from hoisting 2 * LPW of them out of the loop, where they would
-    // be spilled).
-    int ln = lane;
-    if constexpr (kLean) asm volatile("" : "+v"(ln));
     // The wave's first 1 KiB block of the tile, recomputed at every fetch (an opaque copy of the
     // wave index): hoisted out of the loop, the 2 * LPW LDS addresses would occupy scalar
     // registers for the whole loop and be spilled.
@@ -565,11 +693,11 @@ __global__ __launch_bounds__(64 * W) void prefill_mfma_kernel(PrefillArgs a) {
     asm volatile("" : "+s"(wblk));
     // Byte offsets of this lane's chunk of the wave's block i (1 KiB) of the tile in K and V. The
     // chunk's tile row has low four bits bw | RPB i | q (bw: those of the wave's first block, a
-    // multiple of RPB LPW; q = ln / CPR; disjoint bit fields), and both swizzles are XOR-linear in
+    // multiple of RPB LPW; q = lane / CPR; disjoint bit fields), and both swizzles are XOR-linear in
     // those bits, so each offset is a lane term, computed once per fetch, combined with a term of
     // i alone (an XOR-add and a scalar add per load, no 32-bit multiply).
-    const int q = int(uint32_t(ln) / CPR);
-    const int slot = int(uint32_t(ln) % CPR);
+    const int q = lane / CPR;
+    const int slot = lane % CPR;
     const int bw = (wblk * RPB) & 15;
     const uint32_t lane_hi = __umul24(uint32_t(bw | q), row_bytes);
     const uint32_t lane_k = uint32_t(slot ^ lds_swizzle(bw | q)) * 16u;
@@ -580,28 +708,15 @@ __global__ __launch_bounds__(64 * W) void prefill_mfma_kernel(PrefillArgs a) {
       off_k = ((lane_k ^ uint32_t(16 * lds_swizzle(RPB * i))) + lane_hi) + ri;
       off_v = ((lane_v ^ uint32_t(16 * lds_swizzle_v(RPB * i))) + lane_hi) + ri;
     };
-    if constexpr (kAsmLoads) {
-      const u32x4 rk = rsrc_words(at_bytes(a.k_cache, off), nbytes);
-      const u32x4 rv = rsrc_words(at_bytes(a.v_cache, off), nbytes);
+    const u32x4 rk = rsrc_words(at_bytes(a.k_cache, off), nbytes);
+    const u32x4 rv = rsrc_words(at_bytes(a.v_cache, off), nbytes);
 #pragma unroll
-      for (int i = 0; i < LPW; ++i) {
-        const int blk = wblk + i;                  // 1 KiB block of the tile (uniform)
-        uint32_t off_k, off_v;
-        chunk_offsets(i, off_k, off_v);
-        load_lds16(rk, off_k, sk + blk * 512);
-        load_lds16(rv, off_v, sv + blk * 512);
-      }
-    } else {
-      const __amdgpu_buffer_rsrc_t rk = make_rsrc(at_bytes(a.k_cache, off), nbytes);
-      const __amdgpu_buffer_rsrc_t rv = make_rsrc(at_bytes(a.v_cache, off), nbytes);
-#pragma unroll
-      for (int i = 0; i < LPW; ++i) {
-        const int blk = wblk + i;
-        uint32_t off_k, off_v;
-        chunk_offsets(i, off_k, off_v);
-        __builtin_amdgcn_raw_ptr_buffer_load_lds(rk, (lds_ptr_t)(sk + blk * 512), 16, off_k, 0, 0, 0);
-        __builtin_amdgcn_raw_ptr_buffer_load_lds(rv, (lds_ptr_t)(sv + blk * 512), 16, off_v, 0, 0, 0);
-      }
+    for (int i = 0; i < LPW; ++i) {
+      const int blk = wblk + i;                  // 1 KiB block of the tile (uniform)
+      uint32_t off_k, off_v;
+      chunk_offsets(i, off_k, off_v);
+      load_lds16(rk, off_k, sk + blk * 512);
+      load_lds16(rv, off_v, sv + blk * 512);
     }
   };
 
@@ -626,30 +741,13 @@ __global__ __launch_bounds__(64 * W) void prefill_mfma_kernel(PrefillArgs a) {
           return *reinterpret_cast<const u32x4*>(sk + (16 * j + n) * D +
                                                 (((4 * kk + g) ^ lds_swizzle(n)) * 8));
         };
-        if constexpr (kLean) {
-          // K reads two k-steps ahead of their MFMAs (a ring of three operands).
-          u32x4 kop[3];
-          kop[0] = read_k(0);
-          kop[1] = read_k(1);
+        u32x4 kop[KK];
 #pragma unroll
-          for (int kk = 0; kk < KK; ++kk) {
-            __builtin_amdgcn_sched_barrier(0);
-            if (kk + 2 < KK) kop[(kk + 2) % 3] = read_k(kk + 2);
+        for (int kk = 0; kk < KK; ++kk) kop[kk] = read_k(kk);
 #pragma unroll
-            for (int c = 0; c < C; ++c) {
-              s[j][c] = mfma16x16x32(kop[kk % 3], qop[c][kk], s[j][c], Tag{});
-            }
-          }
-          __builtin_amdgcn_sched_barrier(0);
-        } else {
-          u32x4 kop[KK];
+        for (int kk = 0; kk < KK; ++kk) {
 #pragma unroll
-          for (int kk = 0; kk < KK; ++kk) kop[kk] = read_k(kk);
-#pragma unroll
-          for (int kk = 0; kk < KK; ++kk) {
-#pragma unroll
-            for (int c = 0; c < C; ++c) s[j][c] = mfma16x16x32(kop[kk], qop[c][kk], s[j][c], Tag{});
-          }
+          for (int c = 0; c < C; ++c) s[j][c] = mfma16x16x32(kop[kk], qop[c][kk], s[j][c], Tag{});
         }
       }
     }
@@ -685,31 +783,31 @@ __global__ __launch_bounds__(64 * W) void prefill_mfma_kernel(PrefillArgs a) {
           }
         }
       }
-      float mx = v[0];
+      float mx = max2(v[0], v[1]);
 #pragma unroll
-      for (int i = 1; i < 4 * NS; ++i) mx = fmaxf(mx, v[i]);
-      mx = row_group_max(mx) * a.scale_log2;
+      for (int i = 2; i < 4 * NS; i += 2) mx = max3(mx, v[i], v[i + 1]);
       // The running maximum (exp2 units) moves only when the tile's maximum exceeds it by more
       // than kRescaleSlack: P then stays <= 2^kRescaleSlack and O is rescaled rarely. Which
-      // maximum is used cancels in O / l; it only sets the scale at which P is rounded.
-      const bool grow = mx > m_run[c] + kRescaleSlack;
-      const float m_next = grow ? mx : m_run[c];
-      const float alpha = grow ? fast_exp2(m_run[c] - m_next) : 1.f;
-      const float m_use = (m_next == -INFINITY) ? 0.f : m_next;
+      // maximum is used cancels in O / l; it only sets the scale at which P is rounded. Unless some
+      // lane's score asks for it, the rows' maxima need not even be formed across their four lanes.
+      if (__builtin_amdgcn_ballot_w64(mx * a.scale_log2 > m_run[c] + kRescaleSlack) != 0) {
+        mx = row_group_max(mx) * a.scale_log2;
+        const bool grow = mx > m_run[c] + kRescaleSlack;
+        const float m_next = grow ? mx : m_run[c];
+        const float alpha = grow ? fast_exp2(m_run[c] - m_next) : 1.f;
+        l_run[c] *= alpha;
+        m_run[c] = m_next;
+#pragma unroll
+        for (int i = 0; i < NT; ++i) o[c][i] *= alpha;
+      }
+      const float m_use = (m_run[c] == -INFINITY) ? 0.f : m_run[c];
       float p[4 * NS];
 #pragma unroll
       for (int i = 0; i < 4 * NS; ++i) p[i] = fast_exp2(fmaf(v[i], a.scale_log2, -m_use));
-      float psum = 0.f;
 #pragma unroll
       for (int h = 0; h < NS / 2; ++h) {
-        psum += ((p[8 * h] + p[8 * h + 1]) + (p[8 * h + 2] + p[8 * h + 3])) +
-                ((p[8 * h + 4] + p[8 * h + 5]) + (p[8 * h + 6] + p[8 * h + 7]));
-      }
-      l_run[c] = l_run[c] * alpha + psum;
-      m_run[c] = m_next;
-      if (__builtin_amdgcn_ballot_w64(grow) != 0) {
-#pragma unroll
-        for (int i = 0; i < NT; ++i) o[c][i] *= alpha;
+        l_run[c] += ((p[8 * h] + p[8 * h + 1]) + (p[8 * h + 2] + p[8 * h + 3])) +
+                    ((p[8 * h + 4] + p[8 * h + 5]) + (p[8 * h + 6] + p[8 * h + 7]));
       }
 #pragma unroll
       for (int h = 0; h < NS / 2; ++h) {
@@ -735,16 +833,8 @@ __global__ __launch_bounds__(64 * W) void prefill_mfma_kernel(PrefillArgs a) {
       const uint16_t* svh = sv + 32 * h * D;
       auto read_v = [&](int dt) __attribute__((always_inline)) {
         const int dh = dt >> 3, dl = dt & 7;
-        int o0, o1;
-        if constexpr (kLean) {
-          o0 = vbase[0] + ((16 * dl) ^ vxor[0]);
-          o1 = vbase[1] + ((16 * dl) ^ vxor[1]);
-        } else {
-          o0 = voff[0][dl];
-          o1 = voff[1][dl];
-        }
-        const u32x2 lo = lds_read_tr4(svh + o0 + 128 * dh);
-        const u32x2 hi = lds_read_tr4(svh + o1 + 128 * dh);
+        const u32x2 lo = lds_read_tr4(svh + voff[0][dl] + 128 * dh);
+        const u32x2 hi = lds_read_tr4(svh + voff[1][dl] + 128 * dh);
         return u32x4{lo[0], lo[1], hi[0], hi[1]};
       };
       u32x4 vop[3];
@@ -772,14 +862,9 @@ __global__ __launch_bounds__(64 * W) void prefill_mfma_kernel(PrefillArgs a) {
   // Attention of unit (b, kvh, qr0) over its key tiles [t0, t1): leaves the unnormalised o and
   // the per-lane m_run / l_run. Uniform over the workgroup.
   auto run_unit = [&](int t0, int t1) __attribute__((always_inline)) {
-    sx = seq_extent(a, b);
-    sx.q_start = __builtin_amdgcn_readfirstlane(sx.q_start);
-    sx.q_len = __builtin_amdgcn_readfirstlane(sx.q_len);
-    sx.kv_len = __builtin_amdgcn_readfirstlane(sx.kv_len);
-    sx.offset = __builtin_amdgcn_readfirstlane(sx.offset);
     // Rows of the unit: ROWS (per-unit) or its query block's tokens (balanced), clipped to the
     // sequence's rows.
-    const int ur = min(a.balanced_wgs > 0 ? a.tq * G : ROWS, sx.q_len * G - qr0);
+    const int ur = min(BAL ? a.tq * G : ROWS, sx.q_len * G - qr0);
 #pragma unroll
     for (int c = 0; c < C; ++c) {
       const int rho = wave * 16 * C + 16 * c + n;
@@ -813,12 +898,10 @@ __global__ __launch_bounds__(64 * W) void prefill_mfma_kernel(PrefillArgs a) {
     // Q lands here, before the tile loads are issued: the compiler does not see loads issued as
     // assembly, and its wait for Q at the first use, inside the tile loop, would also wait for
     // them.
-    if constexpr (kAsmLoads) {
 #pragma unroll
-      for (int c = 0; c < C; ++c) {
+    for (int c = 0; c < C; ++c) {
 #pragma unroll
-        for (int kk = 0; kk < KK; ++kk) asm volatile("" : "+v"(qop[c][kk]));
-      }
+      for (int kk = 0; kk < KK; ++kk) asm volatile("" : "+v"(qop[c][kk]));
     }
     if (cnt > 0) {
       fetch(sk0, sv0, 0, t0 * kKT);
@@ -909,91 +992,671 @@ __global__ __launch_bounds__(64 * W) void prefill_mfma_kernel(PrefillArgs a) {
 
   // Work of this workgroup: one unit, or (balanced) a run of key tiles over consecutive units.
   // One call site per lambda keeps every per-lane array in registers.
-  const bool balanced = a.balanced_wgs > 0;
-  // Balanced runs are dealt to the XCDs in contiguous blocks: workgroup ids go round-robin over
-  // the 8 XCDs, so run i = (id % 8) * (G / 8) + id / 8 keeps consecutive runs (one KV head,
-  // query blocks of one sequence, the same K/V pages) in one XCD's L2.
-  const int nwg = a.balanced_wgs;
-  const int i = (nwg % kXcds == 0) ? int(blockIdx.x % kXcds) * (nwg / kXcds) + int(blockIdx.x / kXcds)
-                                   : int(blockIdx.x);
-  const PlanView v = plan_view(a);
-  int p = 0, n_pairs = 1, grid_nt = 0, unit_work = 1;
-  int64_t pos = 0, end = 0;  // this workgroup's work positions (balanced)
-  int grid_t0 = 0;  // per-unit schedule: the key tiles [grid_t0, grid_nt) of this workgroup
-  if (!balanced) {
+  if constexpr (BAL) {
+    __shared__ Walk s_walk[W];
+    Walk& w = s_walk[wave];
+    if (!walk_start(a, w)) return;  // uniform over the workgroup
+    do {
+      b = uni(w.b);
+      kvh = uni(w.kvh);
+      qr0 = uni(w.qr0);
+      sx = walk_extent(w);
+      run_unit(uni(w.t0), uni(w.t1));
+      // Units without keys get their zero rows from the merge.
+      if (uni(w.whole) != 0) store_final();
+      else store_partial((int64_t(run_index(a)) * 2 + (uni(w.slot0) ? 0 : 1)) * ROWS);
+    } while (uni(w.fin) == 0 && walk_next(a, w));
+  } else {
     // The heaviest query blocks (latest tokens, longest causal range) are dispatched first.
     kvh = blockIdx.x;
     b = blockIdx.z / a.key_splits;
     split = blockIdx.z - b * a.key_splits;
     qr0 = (gridDim.y - 1 - blockIdx.y) * ROWS;
-    const SeqExtent s0 = seq_extent(a, b);
-    if (qr0 >= s0.q_len * G) return;  // uniform over the workgroup
-    grid_nt = (rows_key_end(a, s0, qr0, ROWS) + kKT - 1) / kKT;
+    sx = seq_extent(a, b);
+    sx.q_start = uni(sx.q_start);
+    sx.q_len = uni(sx.q_len);
+    sx.kv_len = uni(sx.kv_len);
+    sx.offset = uni(sx.offset);
+    if (qr0 >= sx.q_len * G) return;  // uniform over the workgroup
+    int t0 = 0;  // the key tiles [t0, t1) of this workgroup
+    int t1 = (rows_key_end(a, sx, qr0, ROWS) + kKT - 1) / kKT;
     if (a.key_splits > 1) {
-      const int per = (grid_nt + a.key_splits - 1) / a.key_splits;
-      grid_t0 = min(split * per, grid_nt);
-      grid_nt = min(grid_t0 + per, grid_nt);
+      const int per = (t1 + a.key_splits - 1) / a.key_splits;
+      t0 = min(split * per, t1);
+      t1 = min(t0 + per, t1);
     }
-  } else {
-    p = __builtin_amdgcn_readfirstlane(v.wg_p[i]);
-    if (p < 0) return;  // no work left for this workgroup
-    kvh = __builtin_amdgcn_readfirstlane(v.wg_kvh[i]);
-    n_pairs = __builtin_amdgcn_readfirstlane(v.hdr[0]);
-    unit_work = __builtin_amdgcn_readfirstlane(v.hdr[1]);
-    const int64_t runs = __builtin_amdgcn_readfirstlane(v.hdr[2]);
-    const int64_t total = __builtin_amdgcn_readfirstlane(v.hdr[3]);
-    pos = int64_t(i) * total / runs;
-    end = int64_t(i + 1) * total / runs;
+    run_unit(t0, t1);
+    store_final();  // (a key split's unnormalised part, into its slot)
   }
-  // A run that starts inside a unit defers that first piece (the unit's tail) to its end: every
-  // run then starts at key 0 of a unit, and the deferred tail begins about where the run's last
-  // piece (the next unit's head, same cut) ended, so an XCD's workgroups sweep the keys together
-  // and share pages in L2. Partial slot 0 stays the run's first piece, slot 1 its last.
-  bool first = true, deferred = false, replay = false;
-  int d_p = 0, d_kvh = 0;
+}
+
+// A workgroup's rows are the (token, query head) pairs of one KV head's group, row = token * group
+// + head-in-group: 64 C rows, 16 C of them for each of four wave pairs. The two waves of a pair
+// share a SIMD and split the work of their rows: the score wave (waves 0-3) holds Q, computes
+// S^T = K.Q^T and the online softmax of a key tile and leaves P^T in LDS, in the MFMA operand
+// layout, with the factors by which O has to be rescaled; one step later the output wave (waves
+// 4-7) adds V^T.P^T of that tile to the O it holds. A SIMD thus always has the MFMAs of P.V to run
+// beside the softmax, and every K or V operand read from LDS feeds C MFMAs: with O and Q in
+// different waves C = 3 column tiles fit the 256 registers of two waves per SIMD at head_dim 256,
+// where one wave holding both has room for one.
+//
+// K/V tiles of 32 keys go from the pages straight into LDS (buffer loads with the LDS
+// destination), K by the score waves two steps ahead of their use, V by the output waves as far
+// ahead, into rings of three stages each. One barrier per step publishes the tile of K, the tile
+// of V and the P^T of the step before. LDS rows are unpadded and swizzled (lds_swizzle) so that
+// the MFMA operand reads are free of bank conflicts.
+// P2: page_size is a power of two (page_shift >= 0); pages are then found with shifts (a runtime
+// division costs ~20 scalar instructions).
+// SMALL: pages of 4 or 8 tokens (P2 as well). A 16-key sub-tile then spans 16 / page_size pages:
+// each 1 KiB load (2 or 4 rows) lies in one page and gets that page's descriptor, and the keys
+// present in a tile are a bit mask (an absent page can share a sub-tile with a present one).
+//
+// What bounds it: on long runs the card's power limit. A continuation of 2,048 tokens over 8,192 keys
+// runs at 2.0 GHz (of 2.4) with the matrix cores busy 56 % of the cycles (2,726 a step, both waves
+// of a pair busy for 2,420 to 2,550 of them). Against the form before (12 waves of 16 rows, each
+// holding Q and O of its rows and reading every K and V operand for them alone: 2.7 times the LDS
+// reads), whole calls on one box: that continuation 363 -> 323 us, an 8,192-token prompt
+// 796 -> 712, six ragged chunks with context 257 -> 243, eight chunks of 16 over 8,000 keys
+// 75 -> 68; units of a few tiles are even (24 prompts of 17 to 700 tokens 130 -> 130).
+// Why three stages of K and five of V: the loads of a tile are issued two steps before its scores
+// and land within one; V is read two steps after K. 192 rows take all 160 KiB so. Where in the step
+// the loads are issued makes no difference (within 2 %).
+constexpr int kKeyTile = 32;   // keys per staged tile
+constexpr int kKStages = 3;    // tiles of K in LDS
+constexpr int kVStages = 5;    // tiles of V in LDS
+constexpr int kPairs = 4;      // wave pairs of a workgroup
+
+// Where a wave's rows of a tile lie in the caches, for the wave that loads them: byte offset (two
+// words) and bytes that exist from there (the fourth word is unused). Pages of 4 tokens split the
+// wave's kKeyTile / kPairs rows over two pages, so there are two.
+typedef u32x4 RowsAt;
+
+// Walks the tiles of a workgroup, ahead of their computation, and describes for wave `pair` of four
+// the rows of each that it loads (kKeyTile / kPairs of them, inside one 16-key sub-tile).
+template <int D, bool P2, bool SMALL>
+struct TileFinder {
+  static constexpr int RPW = kKeyTile / kPairs;  // rows of a tile a wave loads
+  static_assert(RPW == 8, "a wave's rows lie inside one sub-tile and in at most two pages");
+
+  bool live;        // there is a tile
+  int tile, t1;     // it, in key tiles of the current piece's unit, and the piece's end
+  int kv_len;       // of the current piece's sequence
+  uint32_t head;    // byte offset of its KV head in a cache row
+  const int32_t* bt_row;
+  // Lane l holds the block id of the tile's key l % 32, requested a step ahead of its use. (A
+  // vector load: it is counted apart from the LDS accesses of the score wave, which has no other
+  // vector loads in its tile loop.)
+  int id;
+
+  // The first tile of the walk's piece.
+  __device__ __forceinline__ void enter(const PrefillArgs& a, const Walk& w, int lane) {
+    live = true;
+    tile = uni(w.t0);
+    t1 = uni(w.t1);
+    head = uint32_t(uni(w.kvh)) * uint32_t(D * 2);
+    const int b = uni(w.b);
+    kv_len = uni(w.kv_len);
+    bt_row = a.block_table + int64_t(b) * a.bt_stride;
+    request(a, lane);
+  }
+
+  // Requests the ids of tile `tile` (past the context the last page's id is read and left out; a
+  // piece has at least one key).
+  __device__ __forceinline__ void request(const PrefillArgs& a, int lane) {
+    const uint32_t key = uint32_t(min(tile * kKeyTile + (lane & (kKeyTile - 1)), kv_len - 1));
+    id = bt_row[P2 ? key >> a.page_shift : key / uint32_t(a.page_size)];
+  }
+
+  // `rows` rows from byte `at` of page `page` (nothing for an id outside the cache). A page's bytes
+  // fit 32 bits (the host refuses larger pages), so its byte offset is one 32 x 32-bit product.
+  __device__ __forceinline__ RowsAt rows_at(const PrefillArgs& a, int page, uint32_t at,
+                                            int rows) const {
+    const bool gone = uint32_t(page) >= uint32_t(a.num_blocks32) || rows <= 0 || !live;
+    const uint32_t row_bytes = uint32_t(a.row_stride) * 2u;
+    const uint64_t off =
+        uint64_t(uint32_t(gone ? 0 : page)) * (uint32_t(a.page_stride) * 2u) + (at + head);
+    return RowsAt{uint32_t(off), uint32_t(off >> 32),
+                  gone ? 0u : uint32_t(rows - 1) * row_bytes + D * 2, 0u};
+  }
+
+  // Describes the tile, returns its present keys (bit i: key i is inside the context and its page
+  // id valid), moves to the next tile and requests its ids. Without branches, so that it can ride
+  // between MFMAs.
+  __device__ __forceinline__ uint32_t describe(const PrefillArgs& a, int pair, int lane,
+                                               RowsAt (&out)[2]) {
+    const int k0 = tile * kKeyTile;
+    const uint32_t have = uint32_t(__builtin_amdgcn_ballot_w64(
+        live & (k0 + (lane & (kKeyTile - 1)) < kv_len) & (uint32_t(id) < uint32_t(a.num_blocks32))));
+    const uint32_t row_bytes = uint32_t(a.row_stride) * 2u;
+    const int key = k0 + RPW * pair;
+    const int first = __builtin_amdgcn_readlane(id, RPW * pair);
+    if constexpr (SMALL) {
+      const int ps = a.page_size;
+      out[0] = rows_at(a, first, 0u, min(kv_len - key, ps));
+      out[1] = rows_at(a, __builtin_amdgcn_readlane(id, RPW * pair + 4), 0u,
+                       ps == 4 ? min(kv_len - key - 4, ps) : 0);
+    } else {
+      const uint32_t in_page = P2 ? uint32_t(key) & uint32_t(a.page_size - 1)
+                                  : uint32_t(key) % uint32_t(a.page_size);
+      out[0] = rows_at(a, first, in_page * row_bytes, min(kv_len - key, RPW));
+    }
+    ++tile;
+    request(a, lane);
+    return have;
+  }
+
+  // After `describe`: where that tile was its piece's last, goes to the next piece's first.
+  __device__ __forceinline__ void settle(const PrefillArgs& a, Walk& w, int lane) {
+    if (live && tile == t1) {  // uniform
+      live = uni(w.fin) == 0 && walk_next(a, w);
+      if (live) enter(a, w, lane);
+    }
+  }
+};
+
+template <int D, int C, bool P2, bool SMALL, typename Tag>
+__global__ __launch_bounds__(128 * kPairs) void prefill_pair_kernel(PrefillArgs a) {
+  constexpr int KK = D / 32;
+  constexpr int NT = D / 16;
+  constexpr int ROWS = 16 * C * kPairs;
+  constexpr int TILE = kKeyTile * D;  // elements of a staged tile
+  typedef TileFinder<D, P2, SMALL> Finder;
+  constexpr int RPB = 1024 / (2 * D);       // rows per 1 KiB load (64 lanes x 16 bytes)
+  constexpr int CPR = D / 8;                // 16-byte chunks per row
+  constexpr int LPW = Finder::RPW / RPB;    // 1 KiB loads per loading wave and tile, each of K and V
+
+  __shared__ __align__(1024) uint16_t s_k[kKStages * TILE];
+  __shared__ __align__(1024) uint16_t s_v[kVStages * TILE];
+  // Handed from a score wave to its output wave, by parity of the tile: P^T, the factors of O's
+  // rows and whether the tile is to be skipped (2) or O rescaled (1); at the end of a piece each
+  // row's (m, l).
+  __shared__ u32x4 s_p[2][kPairs][C][64];
+  __shared__ float s_alpha[2][kPairs][C][16];
+  __shared__ int s_flag[2][kPairs];
+  __shared__ float s_ml[2][kPairs][C][2][16];
+  // Handed from a score wave to its output wave, which loads K and V: where its rows of the tiles
+  // to come lie.
+  __shared__ RowsAt s_rows[4][kPairs][SMALL ? 2 : 1];
+  // Each wave's walk over the tiles it computes, then the score waves' over those they describe.
+  __shared__ Walk s_walk[3 * kPairs];
+
+  const int lane = threadIdx.x & 63;
+  const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
+  const int pair = wave & (kPairs - 1);
+  const int n = lane & 15;
+  const int g = lane >> 4;
+  const int G = a.group;
+
+  Walk& w = s_walk[wave];
+  if (!walk_start(a, w)) return;  // uniform over the workgroup
+
+  // Rows of the piece's unit: its query block's tokens, clipped to the sequence's rows.
+  auto unit_rows = [&](const SeqExtent& sx) __attribute__((always_inline)) {
+    return min(a.tq * G, sx.q_len * G - uni(w.qr0));
+  };
+  auto extent = [&]() __attribute__((always_inline)) { return walk_extent(w); };
+
+  if (wave < kPairs) {
+    // ---- Score wave -----------------------------------------------------------------------------
+    SeqExtent sx;
+    int wave_last_key, wave_first_key;
+    bool row_ok[C];
+    int q_pos[C];
+    u32x4 qop[C][KK];
+    int tile = 0, t_end = 0;
+    auto enter = [&]() __attribute__((always_inline)) {
+      sx = extent();
+      const int ur = unit_rows(sx);
+      const int qr0 = uni(w.qr0);
+      const int kvh = uni(w.kvh);
+#pragma unroll
+      for (int c = 0; c < C; ++c) {
+        const int rho = pair * 16 * C + 16 * c + n;
+        const int tok = (qr0 + rho) / G;  // token of the row within the sequence
+        const int hh = qr0 + rho - tok * G;
+        row_ok[c] = rho < ur;
+        q_pos[c] = a.causal ? sx.offset + tok : INT32_MAX;
+        const uint16_t* qrow = a.q + int64_t(sx.q_start + tok) * a.q_st +
+                               int64_t(kvh * G + hh) * a.q_sh + 8 * g;
+#pragma unroll
+        for (int kk = 0; kk < KK; ++kk) {
+          qop[c][kk] = row_ok[c] ? load16(qrow + 32 * kk) : u32x4{0u, 0u, 0u, 0u};
+        }
+      }
+      // Under the causal mask, keys past wave_last_key are masked for every row of the wave and
+      // keys up to wave_first_key are visible to all of them. A wave without rows sees none.
+      const int wave_row = min(ur - 1, (pair + 1) * 16 * C - 1);
+      const bool some = pair * 16 * C < ur;
+      wave_last_key = !some ? -1 : a.causal ? sx.offset + (qr0 + wave_row) / G : INT32_MAX;
+      wave_first_key = a.causal ? sx.offset + (qr0 + pair * 16 * C) / G : INT32_MAX;
+      tile = uni(w.t0);
+      t_end = uni(w.t1);
+    };
+    // K operand addresses: row n, 16-byte chunk 4 kk + g of the swizzled row; k-steps 4 apart and
+    // the two sub-tiles differ by constants.
+    constexpr int KR = 4;
+    const float move_scale = 1.f / a.scale_log2;
+    int koff[4];
+#pragma unroll
+    for (int i = 0; i < 4; ++i) koff[i] = n * D + ((4 * i + g) ^ lds_swizzle(n)) * 8;
+    // Two tiles' scores, the last computed one and the one before (masked; -inf before the first).
+    f32x4 sa[2][C], sb[2][C];
+    // Each row's running maximum (exp2 units) as the term -m of its exponents (0 for none yet) and
+    // the score above which it moves; the lane's part of the denominator.
+    float neg_m[C], m_move[C], l_run[C];
+    auto reset_ml = [&](int c) __attribute__((always_inline)) {
+      neg_m[c] = 0.f;
+      m_move[c] = -INFINITY;
+      l_run[c] = 0.f;
+    };
+#pragma unroll
+    for (int c = 0; c < C; ++c) {
+      sb[0][c] = sb[1][c] = f32x4{-INFINITY, -INFINITY, -INFINITY, -INFINITY};
+      reset_ml(c);
+    }
+    bool cur = true;          // this step has a tile
+    bool prev_vis = false;    // the tile before holds a key that some row of the wave can see
+    bool prev_last = false;   // and is the last of its piece
+    int stage = 0;            // of this step's tile
+    // In step s the rows of tile s + 4 are described; the output wave takes them up in step s + 1
+    // and issues their loads in step s + 2. have: the present keys of tiles s .. s + 3.
+    Walk& wf = s_walk[2 * kPairs + wave];
+    wf = w;
+    Finder fd;
+    fd.enter(a, wf, lane);
+    int at_rows = 0;
+    auto find = [&]() __attribute__((always_inline)) {
+      RowsAt r[2];
+      const uint32_t h = fd.describe(a, pair, lane, r);
+      s_rows[at_rows][pair][0] = r[0];
+      if constexpr (SMALL) s_rows[at_rows][pair][SMALL ? 1 : 0] = r[1];
+      at_rows = (at_rows + 1) & 3;
+      return h;
+    };
+    uint32_t have[4];
+#pragma unroll
+    for (int i = 0; i < 4; ++i) {
+      have[i] = find();
+      fd.settle(a, wf, lane);
+    }
+    enter();
+    asm volatile("s_waitcnt lgkmcnt(0)\n\ts_barrier" ::: "memory");
+    // The score wave's chain (operand reads, MFMAs, softmax, hand-over) is the step's longest;
+    // the output wave fills the matrix core where it leaves it free.
+    __builtin_amdgcn_s_setprio(2);
+    // One step: S^T of this step's tile into s; the softmax of the tile before, whose scores are
+    // v, with P^T handed over in the slots of parity par. Returns whether it was the drain step
+    // after the last tile (whose MFMAs' results are not used).
+    auto run_step = [&](f32x4 (&v)[2][C], f32x4 (&s)[2][C], const int par)
+        __attribute__((always_inline)) -> bool {
+      // K of this step's tile is in LDS (the loading waves have waited for it).
+      asm volatile("s_waitcnt lgkmcnt(0)\n\ts_barrier" ::: "memory");
+      const uint16_t* sk = s_k + stage * TILE;
+      auto read_k = [&](int i) __attribute__((always_inline)) {  // k-step i / 2, sub-tile i % 2
+        return *reinterpret_cast<const u32x4*>(sk + koff[(i >> 1) & 3] + 128 * (i >> 3) +
+                                              16 * D * (i & 1));
+      };
+      // The MFMAs and the softmax run in one straight sequence of 2 KK slots: each holds one K
+      // operand read (KR - 1 slots ahead of its use), its C MFMAs and a share of the softmax, which
+      // runs in the MFMAs' shadow. The scheduling barriers keep that order.
+      u32x4 kop[KR];
+#pragma unroll
+      for (int i = 0; i < KR - 1; ++i) kop[i] = read_k(i);
+      auto mfma_slot = [&](int i) __attribute__((always_inline)) {
+        __builtin_amdgcn_sched_barrier(0);
+        if (i + KR - 1 < 2 * KK) kop[(i + KR - 1) % KR] = read_k(i + KR - 1);
+#pragma unroll
+        for (int c = 0; c < C; ++c) {
+          s[i & 1][c] = mfma16x16x32(kop[i % KR], qop[c][i >> 1],
+                                     i < 2 ? f32x4{0.f, 0.f, 0.f, 0.f} : s[i & 1][c], Tag{});
+        }
+      };
+      // Slots 0 and 1: each lane's largest score per column tile.
+      float mx[C];
+      bool up = false;
+#pragma unroll
+      for (int i = 0; i < 2; ++i) {
+        mfma_slot(i);
+#pragma unroll
+        for (int c = (C * i) / 2; c < (C * (i + 1)) / 2; ++c) {
+          mx[c] = max3(max3(max3(v[0][c][0], v[0][c][1], v[0][c][2]), v[0][c][3], v[1][c][0]),
+                       v[1][c][1], max2(v[1][c][2], v[1][c][3]));
+          up |= mx[c] > m_move[c];
+        }
+      }
+      // The running maximum moves only when the tile's maximum exceeds it by more than
+      // kRescaleSlack: P then stays <= 2^kRescaleSlack and O is rescaled rarely. Which maximum is
+      // used cancels in O / l; it only sets the scale at which P is rounded. Unless some lane's
+      // score asks for it, the rows' maxima need not even be formed across their four lanes.
+      const bool grown = __builtin_amdgcn_ballot_w64(up) != 0;
+      if (grown) {  // uniform
+#pragma unroll
+        for (int c = 0; c < C; ++c) {
+          const float m_row = row_group_max(mx[c]) * a.scale_log2;
+          const bool grow = row_group_max(mx[c]) > m_move[c];
+          const bool none = m_move[c] == -INFINITY;
+          const float alpha = grow ? (none ? 0.f : fast_exp2(-neg_m[c] - m_row)) : 1.f;
+          if (grow) {
+            neg_m[c] = -m_row;
+            m_move[c] = (m_row + kRescaleSlack) * move_scale;
+          }
+          l_run[c] *= alpha;
+          s_alpha[par][pair][c][n] = alpha;  // the row's four lanes write the same value
+        }
+      }
+      uint32_t have_next = 0;
+      const int k0 = tile * kKeyTile;
+      bool full = false, vis = false, last = false;
+      float p[C][8];
+      // The other slots: part `part` of 5 of column tile c's exponentials, sum and hand-over.
+      auto soften = [&](int c, int part) __attribute__((always_inline)) {
+        if (part < 4) {
+#pragma unroll
+          for (int i = 2 * part; i < 2 * part + 2; ++i) {
+            p[c][i] = fast_exp2(fmaf(v[i >> 2][c][i & 3], a.scale_log2, neg_m[c]));
+          }
+        } else {
+          l_run[c] += ((p[c][0] + p[c][1]) + (p[c][2] + p[c][3])) +
+                      ((p[c][4] + p[c][5]) + (p[c][6] + p[c][7]));
+          u32x4 pop;
+#pragma unroll
+          for (int i = 0; i < 4; ++i) pop[i] = pack2(p[c][2 * i], p[c][2 * i + 1], Tag{});
+          s_p[par][pair][c][lane] = pop;
+        }
+      };
+#pragma unroll
+      for (int i = 2; i < 2 * KK; ++i) {
+        mfma_slot(i);
+#pragma unroll
+        for (int u = (5 * C * (i - 2)) / (2 * KK - 2); u < (5 * C * (i - 1)) / (2 * KK - 2); ++u) {
+          soften(u / 5, u % 5);
+        }
+        // The step's scalar work, in the MFMAs' shadow too.
+        if (i == 3) s_flag[par][pair] = !prev_vis ? 2 : grown ? 1 : 0;
+        if (i == 2 * KK - 4) have_next = find();
+        if (i == 2 * KK - 2) {
+          // A tile wholly below the wave's diagonal with every key present needs no mask (uniform).
+          full = k0 + kKeyTile - 1 <= wave_first_key && have[0] == 0xffffffffu;
+          vis = k0 <= wave_last_key;
+          last = tile + 1 == t_end;
+        }
+      }
+      __builtin_amdgcn_sched_barrier(0);
+      if (prev_last) {  // uniform
+#pragma unroll
+        for (int c = 0; c < C; ++c) {
+          const float l_tot = row_group_sum(l_run[c]);
+          s_ml[par][pair][c][0][n] = m_move[c] == -INFINITY ? -INFINITY : -neg_m[c];
+          s_ml[par][pair][c][1][n] = l_tot;
+          reset_ml(c);
+        }
+      }
+      if (!cur) return true;
+      if (!full) {
+#pragma unroll
+        for (int j = 0; j < 2; ++j) {
+          const uint32_t keys = have[0] >> (16 * j + 4 * g);  // this lane's four, from bit 0
+#pragma unroll
+          for (int c = 0; c < C; ++c) {
+#pragma unroll
+            for (int r = 0; r < 4; ++r) {
+              const bool ok = row_ok[c] & ((keys >> r) & 1) & (k0 + 16 * j + 4 * g + r <= q_pos[c]);
+              s[j][c][r] = ok ? s[j][c][r] : -INFINITY;
+            }
+          }
+        }
+      }
+#pragma unroll
+      for (int i = 0; i < 3; ++i) have[i] = have[i + 1];
+      have[3] = have_next;
+      prev_vis = vis;
+      prev_last = last;
+      ++tile;
+      stage = stage == kKStages - 1 ? 0 : stage + 1;
+      if (prev_last) {
+        cur = uni(w.fin) == 0 && walk_next(a, w);
+        if (cur) enter();
+      }
+      fd.settle(a, wf, lane);
+      return false;
+    };
+    for (;;) {
+      if (run_step(sb, sa, 1)) break;
+      if (run_step(sa, sb, 0)) break;
+    }
+    asm volatile("s_waitcnt lgkmcnt(0)\n\ts_barrier" ::: "memory");  // the last hand-over
+    return;
+  }
+
+  // ---- Output wave --------------------------------------------------------------------------------
+  constexpr int VR = 4;
+  f32x4 o[C][NT];
+  auto clear = [&]() __attribute__((always_inline)) {
+#pragma unroll
+    for (int c = 0; c < C; ++c) {
+#pragma unroll
+      for (int i = 0; i < NT; ++i) o[c][i] = f32x4{0.f, 0.f, 0.f, 0.f};
+    }
+  };
+  clear();
+  // Stores the piece's rows, given each row's (m, l): normalised into `out` (a whole unit), or
+  // unnormalised (o relative to 2^m) into `uo` or the workgroup's partial slot.
+  auto store = [&](const float (&m)[C], const float (&l)[C]) __attribute__((always_inline)) {
+    const SeqExtent sx = extent();
+    const int ur = unit_rows(sx);
+    const int qr0 = uni(w.qr0);
+    const bool whole = uni(w.whole) != 0;
+#pragma unroll
+    for (int c = 0; c < C; ++c) {
+      const int rho = pair * 16 * C + 16 * c + n;
+      if (rho >= ur) continue;
+      const int tok = (qr0 + rho) / G;
+      const int hh = uni(w.kvh) * G + (qr0 + rho - tok * G);
+      if (!whole || a.uo) {  // uniform
+        float *po, *pml;
+        if (whole) {  // unnormalised rows for a later merge
+          const int64_t r = int64_t(sx.q_start + tok) * a.hq + hh;
+          po = a.uo + r * D;
+          pml = a.uml + 2 * r;
+        } else {
+          const int64_t r =
+              (int64_t(run_index(a)) * 2 + (uni(w.slot0) ? 0 : 1)) * ROWS + rho;
+          po = a.part_o + r * D;
+          pml = a.part_ml + 2 * r;
+        }
+#pragma unroll
+        for (int dt = 0; dt < NT; ++dt) {
+          *reinterpret_cast<f32x4*>(po + 16 * dt + 4 * g) = o[c][dt];
+        }
+        if (g == 0) {
+          pml[0] = m[c];
+          pml[1] = l[c];
+        }
+        continue;
+      }
+      uint16_t* orow = a.out + int64_t(sx.q_start + tok) * a.o_st + int64_t(hh) * a.o_sh;
+      const float inv = l[c] > 0.f ? 1.f / l[c] : 0.f;
+      // Lane (n, g) holds d = 16 dt + 4g .. +3 of its row in o[c][dt].
+      const uint16_t* grow = a.gate ? a.gate + int64_t(sx.q_start + tok) * a.gate_st +
+                                          int64_t(hh) * a.gate_sh
+                                    : nullptr;
+#pragma unroll
+      for (int dt = 0; dt < NT; ++dt) {
+        u32x2 x;
+        x[0] = pack2(o[c][dt][0] * inv, o[c][dt][1] * inv, Tag{});
+        x[1] = pack2(o[c][dt][2] * inv, o[c][dt][3] * inv, Tag{});
+        if (grow) {  // uniform
+          const u32x2 gv = *reinterpret_cast<const u32x2*>(grow + 16 * dt + 4 * g);
+          x[0] = gate_mul2(x[0], gv[0], Tag{});
+          x[1] = gate_mul2(x[1], gv[1], Tag{});
+        }
+        *reinterpret_cast<u32x2*>(orow + 16 * dt + 4 * g) = x;
+      }
+    }
+  };
+  // V^T operand addresses for the transposed reads: lane (s, g) (s = lane % 16) points at key row
+  // 16h + 4g + s/4 and columns d0 + 4(s%4) .. +3, so the read gives output lane m the values
+  // V[16h + 4g + i][d0 + m], i = 0..3 -- the k-slots 8g + 4h + i of the A operand (keys 4g + i of
+  // sub-tile h, matching P). The swizzle XORs the 16-byte chunk index 2 dl + ((s % 4) / 2) of
+  // d-tile dl (of 8) with the even 2r & 14, i.e. element offset 16 (dl ^ (r & 7)) + 8 ((s % 4) / 2);
+  // d-tiles 8 apart and the two sub-tiles differ by constants.
+  const int vrow = 4 * g + (n >> 2);
+  const int vbase = vrow * D + ((n & 3) >> 1) * 8 + (n & 1) * 4;
+  const int vxor = 16 * (vrow & 7);
+  // This wave's rows of a tile: block i (1 KiB) of its LPW; this lane's 16-byte chunk of it is
+  // chunk `slot` of tile row first | RPB i | q; both swizzles are XOR-linear in those (disjoint)
+  // bits, so its offset is a lane term combined with a term of i alone.
+  const int lrow = ((pair * Finder::RPW) & 15) | (lane / CPR);
+  const uint32_t row_bytes = uint32_t(a.row_stride) * 2u;
+  const uint32_t lane_k = uint32_t((lane % CPR) ^ lds_swizzle(lrow)) * 16u;
+  const uint32_t lane_v = uint32_t((lane % CPR) ^ lds_swizzle_v(lrow)) * 16u;
+  const uint32_t lane_q = uint32_t(lane / CPR) * row_bytes;
+  int kst = 0, vst = 0;    // stages of the next one
+  int at_rows = 0;
+  u32x4 rk[SMALL ? 2 : 1], rv[SMALL ? 2 : 1];
+  uint16_t *to_k, *to_v;
+  // Takes up the next tile: requests its rows, then forms their descriptors. These span only the
+  // rows that exist, so rows past the context or in an absent page (and everything once no tile is
+  // left) land in LDS as zero without a memory access.
+  RowsAt rows[SMALL ? 2 : 1];
+  auto read_rows = [&]() __attribute__((always_inline)) {
+#pragma unroll
+    for (int j = 0; j < (SMALL ? 2 : 1); ++j) rows[j] = s_rows[at_rows][pair][j];
+  };
+  auto take_rows = [&]() __attribute__((always_inline)) {
+#pragma unroll
+    for (int j = 0; j < (SMALL ? 2 : 1); ++j) {
+      const uint64_t off =
+          uint64_t(uint32_t(uni(int(rows[j][0])))) | uint64_t(uint32_t(uni(int(rows[j][1])))) << 32;
+      const uint32_t nbytes = uint32_t(uni(int(rows[j][2])));
+      rk[j] = rsrc_words(at_bytes(a.k_cache, off), nbytes);
+      rv[j] = rsrc_words(at_bytes(a.v_cache, off), nbytes);
+    }
+    to_k = s_k + kst * TILE + pair * LPW * 512;
+    to_v = s_v + vst * TILE + pair * LPW * 512;
+    at_rows = (at_rows + 1) & 3;
+    kst = kst == kKStages - 1 ? 0 : kst + 1;
+    vst = vst == kVStages - 1 ? 0 : vst + 1;
+  };
+  // Issues load `load` of the tile's 2 LPW (K and V in turn).
+  auto issue = [&](int load) __attribute__((always_inline)) {
+    const int i = load >> 1;
+    uint32_t at = uint32_t(RPB * i) * row_bytes;
+    u32x4 k = rk[0], v = rv[0];
+    if constexpr (SMALL) {
+      const bool second = RPB * i >= 4 && a.page_size == 4;  // uniform
+      if (second) at -= 4u * row_bytes;
+#pragma unroll
+      for (int e = 0; e < 3; ++e) {
+        k[e] = second ? rk[SMALL ? 1 : 0][e] : k[e];
+        v[e] = second ? rv[SMALL ? 1 : 0][e] : v[e];
+      }
+    }
+    // An opaque copy of the lane's term keeps the 2 LPW offsets from being formed ahead of the tile
+    // loop, where they would be spilled.
+    uint32_t x = (load & 1) ? lane_v : lane_k;
+    asm volatile("" : "+v"(x));
+    if ((load & 1) == 0) {
+      load_lds16(k, (x ^ uint32_t(16 * lds_swizzle(RPB * i))) + lane_q + at, to_k + i * 512);
+    } else {
+      load_lds16(v, (x ^ uint32_t(16 * lds_swizzle_v(RPB * i))) + lane_q + at, to_v + i * 512);
+    }
+  };
+  auto issue_all = [&]() __attribute__((always_inline)) {
+#pragma unroll
+    for (int i = 0; i < 2 * LPW; ++i) issue(i);
+  };
+  // In step s the score waves compute S^T of tile s, P^T of tile s - 1 comes into LDS, and tile
+  // s - 2 is added here; the loads of tile s + 2 are issued. Before the barrier of step s, tile s
+  // has landed (this wave's part; the tile after it may be in flight).
+  auto next_step = [&]() __attribute__((always_inline)) {
+    asm volatile("s_waitcnt vmcnt(%0) lgkmcnt(0)\n\ts_barrier" ::"n"(2 * LPW) : "memory");
+  };
+  asm volatile("s_waitcnt lgkmcnt(0)\n\ts_barrier" ::: "memory");  // the first tiles are described
+  read_rows();
+  take_rows();
+#pragma unroll 1
+  for (int i = 0; i < 4; ++i) {
+    if (i >= 2) next_step();
+    issue_all();
+    read_rows();
+    take_rows();
+  }
+  int stage = 0;  // of the tile to add
+  int done = 0;   // its number
   for (;;) {
-    int nt = grid_nt, t0 = grid_t0, t1 = grid_nt;
-    bool last = true;
-    if (balanced) {
-      nt = __builtin_amdgcn_readfirstlane(v.pair_nt[p]);
-      b = __builtin_amdgcn_readfirstlane(v.pair_b[p]);
-      qr0 = __builtin_amdgcn_readfirstlane(v.pair_qb[p]) * a.tq * G;
-      // The unit's key tiles occupy work [k_pos, k_pos + nt); this run covers [pos, end).
-      const int64_t k_pos = int64_t(kvh) * unit_work +
-                            __builtin_amdgcn_readfirstlane(v.pair_pre[p]) + kUnitCost;
-      t0 = int(max(pos - k_pos, int64_t(0)));
-      t1 = int(min(end - k_pos, int64_t(nt)));
-      last = k_pos + nt >= end;
+    // A piece: the tiles that some row of the wave can see, then those that none can.
+    const SeqExtent sx = extent();
+    const int ur = unit_rows(sx);
+    int tile = uni(w.t0);
+    const int t_end = uni(w.t1);
+    int t_vis = pair * 16 * C < ur ? t_end : tile;
+    if (a.causal) {
+      const int last_key =
+          sx.offset + (uni(w.qr0) + min(ur - 1, (pair + 1) * 16 * C - 1)) / G;
+      t_vis = min(t_vis, (last_key >> 5) + 1);
     }
-    const bool slot0 = first || replay;
-    // Units without keys get their zero rows from the merge (balanced) or here (grid: nt = 0).
-    bool go = t0 < t1 || !balanced;
-    if (go && first && t0 > 0 && !last) {  // balanced only (grid units start at 0)
-      d_p = p;
-      d_kvh = kvh;
-      deferred = true;
-      first = false;
-      go = false;
+    for (; tile < t_vis; ++tile) {
+      next_step();
+      const int par = done & 1;
+      const uint16_t* sv = s_v + stage * TILE;
+      auto read_v = [&](int dt) __attribute__((always_inline)) {
+        const uint16_t* vp = sv + (vbase + ((16 * (dt & 7)) ^ vxor)) + 128 * (dt >> 3);
+        const u32x2 lo = lds_read_tr4(vp);
+        const u32x2 hi = lds_read_tr4(vp + 16 * D);
+        return u32x4{lo[0], lo[1], hi[0], hi[1]};
+      };
+      const int flag = s_flag[par][pair];
+      u32x4 pop[C], vop[VR];
+#pragma unroll
+      for (int c = 0; c < C; ++c) pop[c] = s_p[par][pair][c][lane];
+#pragma unroll
+      for (int i = 0; i < VR - 1; ++i) vop[i] = read_v(i);
+      if (uni(flag) == 1) {  // uniform
+#pragma unroll
+        for (int c = 0; c < C; ++c) {
+          const float alpha = s_alpha[par][pair][c][n];
+#pragma unroll
+          for (int i = 0; i < NT; ++i) o[c][i] *= alpha;
+        }
+      }
+#pragma unroll
+      for (int dt = 0; dt < NT; ++dt) {
+        __builtin_amdgcn_sched_barrier(0);
+        if (dt + VR - 1 < NT) vop[(dt + VR - 1) % VR] = read_v(dt + VR - 1);
+#pragma unroll
+        for (int c = 0; c < C; ++c) o[c][dt] = mfma16x16x32(vop[dt % VR], pop[c], o[c][dt], Tag{});
+        // The next loads and the preparation of those after them ride between the MFMAs: a wave
+        // stalls at a load until the texture path takes it, and the MFMAs issued before it run
+        // meanwhile.
+        if (dt * 2 * LPW % NT == 0) issue(dt * 2 * LPW / NT);
+        if (dt == NT - VR) read_rows();
+        if (dt == NT - 1) take_rows();
+      }
+      __builtin_amdgcn_sched_barrier(0);
+      ++done;
+      stage = stage == kVStages - 1 ? 0 : stage + 1;
     }
-    if (go) {
-      run_unit(t0, t1);
-      // Per-unit workgroups store their rows (a key split's unnormalised part, into its slot).
-      if (!balanced || (t0 == 0 && t1 == nt)) store_final();
-      else store_partial((int64_t(i) * 2 + (slot0 ? 0 : 1)) * ROWS);
-      first = false;
+#pragma unroll 1
+    for (; tile < t_end; ++tile) {
+      next_step();
+      issue_all();
+      read_rows();
+      take_rows();
+      ++done;
+      stage = stage == kVStages - 1 ? 0 : stage + 1;
     }
-    bool done = last || replay;
-    if (!done && ++p == n_pairs) {
-      p = 0;
-      done = ++kvh == a.hkv;
+    float m[C], l[C];
+#pragma unroll
+    for (int c = 0; c < C; ++c) {
+      m[c] = s_ml[(done - 1) & 1][pair][c][0][n];
+      l[c] = s_ml[(done - 1) & 1][pair][c][1][n];
     }
-    if (done) {
-      if (!deferred || replay) break;
-      p = d_p;
-      kvh = d_kvh;
-      replay = true;
-    }
+    store(m, l);
+    if (uni(w.fin) != 0 || !walk_next(a, w)) break;
+    clear();
   }
+  asm volatile("s_waitcnt vmcnt(0)" ::: "memory");  // no load may reach LDS after the wave's end
 }
 
 // Combines the partials of every unit that was cut between workgroups, in workgroup order, and
@@ -1111,30 +1774,45 @@ __global__ __launch_bounds__(256) void prefill_merge_kernel(PrefillArgs a) {
   }
 }
 
-// Launch shape per head_dim and schedule: C column tiles per wave, W waves (16 C W rows), NS
-// 16-key sub-tiles per staged tile (each inside one page). head_dim 256, measured in same-process
-// A/Bs on MI355X (config 4, 6 query heads per KV head):
+// Launch shape per head_dim and schedule. prefill_mfma_kernel: C column tiles per wave, W waves (16
+// C W rows), NS 16-key sub-tiles per staged tile (each inside one page). prefill_pair_kernel (W = 0):
+// C column tiles per wave pair (64 C rows), tiles of kKeyTile keys. head_dim 256, measured in
+// same-process A/Bs on MI355X (config 4, 6 query heads per KV head):
 // - one workgroup per unit: 8 waves, 64-key tiles. Units of 128 rows keep a causal first chunk's
-//   longest unit short (82 us for the 2048-token chunk; 12 waves x 192 rows: 106-115 us).
-// - balanced: 12 waves (3 per SIMD, 168 VGPRs), 32-key tiles. 192 rows share each K/V tile, 1.5x
-//   the rows of 8 waves, and the 32-key tile leaves the registers the third wave needs (64-key
-//   tiles spill 22 VGPRs): continuation chunk 405 us against 444 us for 8 waves.
+//   longest unit short (82 us for the 2048-token chunk; 12 waves x 192 rows: 106-115 us). The wave
+//   pairs with 128 rows per workgroup: first chunk 69-71 us against 70-73, but 24 short prompts
+//   127 us against 110 (longer pipeline fill) and the shared-prefix pass 37 against 36.
+// - balanced: wave pairs, 192 rows.
+// head_dim 128: 8 waves, 64-key tiles. The softmax there is twice the work per MFMA, and the score
+// waves of the pairs are bound by it: five ragged chunks 326-328 us (256 rows) against 324.
 template <int D, bool BAL> struct PrefillShape;
 template <> struct PrefillShape<256, false> { static constexpr int C = 1, W = 8, NS = 4; };
-template <> struct PrefillShape<256, true> { static constexpr int C = 1, W = 12, NS = 2; };
+template <> struct PrefillShape<256, true> { static constexpr int C = 3, W = 0, NS = 2; };
 template <bool BAL> struct PrefillShape<128, BAL> { static constexpr int C = 2, W = 8, NS = 4; };
 
+// Rows and threads of a workgroup, and keys of a staged tile.
+template <int D, bool BAL>
+struct PrefillSizes {
+  using S = PrefillShape<D, BAL>;
+  static constexpr bool PAIRS = S::W == 0;
+  static constexpr int ROWS = 16 * S::C * (PAIRS ? kPairs : S::W);
+  static constexpr int THREADS = 64 * (PAIRS ? 2 * kPairs : S::W);
+  static constexpr int KEYS = PAIRS ? kKeyTile : 16 * S::NS;
+};
+
 int prefill_rows(int head_dim, bool balanced) {
-  return head_dim == 256 ? (balanced ? 16 * 1 * 12 : 16 * 1 * 8) : 16 * 2 * 8;
+  return head_dim == 256 ? (balanced ? PrefillSizes<256, true>::ROWS : PrefillSizes<256, false>::ROWS)
+                         : PrefillSizes<128, false>::ROWS;
 }
 int prefill_key_tile(int head_dim, bool balanced) {
-  return head_dim == 256 && balanced ? 16 * 2 : 16 * 4;
+  return head_dim == 256 && balanced ? PrefillSizes<256, true>::KEYS : PrefillSizes<256, false>::KEYS;
 }
 
 template <int D, bool BAL, bool P2, typename Tag, bool SMALL = false>
 constexpr auto prefill_kernel() {
   using S = PrefillShape<D, BAL>;
-  return prefill_mfma_kernel<D, S::C, S::W, S::NS, P2, SMALL, Tag>;
+  if constexpr (S::W == 0) return prefill_pair_kernel<D, S::C, P2, SMALL, Tag>;
+  else return prefill_mfma_kernel<D, S::C, S::W, S::NS, BAL, P2, SMALL, Tag>;
 }
 
 // Workgroups of one balanced launch: every CU's resident workgroups (one round).
@@ -1145,7 +1823,7 @@ int balanced_wgs() {
   if (per_cu == 0) {
     const auto fn = prefill_kernel<D, true, true, Tag>();
     if (hipOccupancyMaxActiveBlocksPerMultiprocessor(&per_cu, reinterpret_cast<const void*>(fn),
-                                                     64 * PrefillShape<D, true>::W, 0) !=
+                                                     PrefillSizes<D, true>::THREADS, 0) !=
             hipSuccess ||
         per_cu <= 0) {
       (void)hipGetLastError();
@@ -1158,29 +1836,30 @@ int balanced_wgs() {
 
 // Upper bound of balanced_wgs (LDS bounds the resident workgroups per CU).
 int balanced_wgs_bound(int head_dim) {
-  const int lds = 4 * prefill_key_tile(head_dim, true) * head_dim * 2;
+  const int tiles = head_dim == 256 ? kKStages + kVStages : 4;  // staged tiles of K and V
+  const int lds = tiles * prefill_key_tile(head_dim, true) * head_dim * 2;
   return device_cu_count() * (160 * 1024 / lds);
 }
 
 template <int D, bool BAL, typename Tag>
 int launch_prefill(const PrefillArgs& a, int batch, int max_q, hipStream_t s) {
-  using S = PrefillShape<D, BAL>;
+  using S = PrefillSizes<D, BAL>;
   const auto kern = a.page_size < 16   ? prefill_kernel<D, BAL, true, Tag, true>()
                     : a.page_shift >= 0 ? prefill_kernel<D, BAL, true, Tag>()
                                         : prefill_kernel<D, BAL, false, Tag>();
   if constexpr (!BAL) {
-    const dim3 grid(unsigned(a.hkv), unsigned(ceil_div(int64_t(max_q) * a.group, S::C * S::W * 16)),
+    const dim3 grid(unsigned(a.hkv), unsigned(ceil_div(int64_t(max_q) * a.group, S::ROWS)),
                     unsigned(batch * a.key_splits));
-    hipLaunchKernelGGL(kern, grid, dim3(64 * S::W), 0, s, a);
+    hipLaunchKernelGGL(kern, grid, dim3(S::THREADS), 0, s, a);
     return check_launch("ti_gqa_prefill_paged");
   } else {
     hipLaunchKernelGGL(prefill_plan_kernel, dim3(1), dim3(kPlanThreads), 0, s, a, batch);
     int rc = check_launch("ti_gqa_prefill_paged (plan)");
     if (rc != TI_OK) return rc;
-    hipLaunchKernelGGL(kern, dim3(unsigned(a.balanced_wgs)), dim3(64 * S::W), 0, s, a);
+    hipLaunchKernelGGL(kern, dim3(unsigned(a.balanced_wgs)), dim3(S::THREADS), 0, s, a);
     rc = check_launch("ti_gqa_prefill_paged");
     if (rc != TI_OK) return rc;
-    constexpr int kRows = 16 * S::C * S::W;
+    constexpr int kRows = S::ROWS;
     constexpr int kMergeRows = 256 / (D / 8) * kMergeRowsPerThread;  // rows per merge workgroup
     static_assert(kRows % kMergeRows == 0, "merge row blocks must tile the unit");
     hipLaunchKernelGGL((prefill_merge_kernel<D, kRows, Tag>),
