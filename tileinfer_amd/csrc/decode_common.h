@@ -51,8 +51,14 @@ __device__ __forceinline__ float2 unpack2(uint32_t v, F16) {
   return make_float2(float(h[0]), float(h[1]));
 }
 
-// Logistic function 1 / (1 + e^-x) through the HIP device library's expf.
-__device__ __forceinline__ float sigmoidf(float x) { return 1.f / (1.f + expf(-x)); }
+// Logistic function 1 / (1 + 2^(-x log2 e)) on the exp2 and reciprocal units (1 ulp each; the scaled
+// argument's rounding adds |x| 2^-24): within 4e-6 relative for |x| <= 40, against the 2^-9 (bf16)
+// or 2^-11 (fp16) of the product it goes into. expf and an IEEE division take ~40 instructions
+// instead of 4, which the epilogue of a gated prefill pays per output value (24 prompts of 17 to
+// 700 tokens: 175 -> 150 us a call).
+__device__ __forceinline__ float sigmoidf(float x) {
+  return __builtin_amdgcn_rcpf(1.f + fast_exp2(-1.4426950408889634f * x));
+}
 
 // a * sigmoid(g) for two packed 16-bit pairs, rounded back to the storage type: the output
 // epilogue of the sigmoid gate (out = attention output * sigmoid(gate)).
