@@ -7,12 +7,15 @@ here). There is no fallback: a missing library raises.
 from __future__ import annotations
 
 import ctypes
+import importlib.machinery
+import importlib.util
 import threading
 from pathlib import Path
 
 import torch  # noqa: F401  (must be imported before the library: shared HIP runtime)
 
 LIB_PATH = Path(__file__).resolve().parent / "libtileinfer_amd.so"
+CALLS_PATH = Path(__file__).resolve().parent / "_pycalls.so"
 
 # Codes mirrored from include/tileinfer_amd.h.
 TI_OK = 0
@@ -133,6 +136,39 @@ def load(path: Path | str | None = None) -> ctypes.CDLL:
         return lib
 
 
+# The library functions that _pycalls.so calls, in the order its bind() takes them.
+_BOUND = ("ti_kv_append", "ti_gqa_decode_plan", "ti_gqa_decode_paged", "ti_gqa_decode_paged_gated",
+          "ti_gqa_decode_paged_append", "ti_gqa_prefill_paged", "ti_gqa_prefill_paged_gated",
+          "ti_gqa_prefill_workspace_bytes", "ti_qknorm_rope_append")
+_calls = None
+
+
+def calls():
+    """The native form of the Python entry points (csrc/pycalls.cpp), bound to the library."""
+    global _calls
+    if _calls is None:
+        lib = load()
+        with _lock:
+            if _calls is None:
+                if not CALLS_PATH.exists():
+                    raise RuntimeError(f"{CALLS_PATH} is missing: build it with "
+                                       "`python -m tileinfer_amd.build`")
+                loader = importlib.machinery.ExtensionFileLoader("_pycalls", str(CALLS_PATH))
+                mod = importlib.util.module_from_spec(
+                    importlib.util.spec_from_loader("_pycalls", loader))
+                loader.exec_module(mod)
+                mod.bind(*(ctypes.cast(getattr(lib, n), ctypes.c_void_p).value for n in _BOUND))
+                _calls = mod
+    return _calls
+
+
+def result(r):
+    """What a function of ``calls()`` returned, its library return codes raised."""
+    if type(r) is int:
+        check(r)
+    return r
+
+
 def check(rc: int) -> None:
     if rc != TI_OK:
         msg = load().ti_last_error().decode(errors="replace")
@@ -148,6 +184,12 @@ def dtype_code(dtype: torch.dtype) -> int:
 
 
 _raw_stream = getattr(torch._C, "_cuda_getCurrentRawStream", None)
+
+
+def current_stream(index: int) -> int:
+    """hipStream_t of torch's current stream on GPU ``index``."""
+    return _raw_stream(index) if _raw_stream is not None else \
+        torch.cuda.current_stream(index).cuda_stream
 
 
 def stream_handle(device: torch.device) -> int:

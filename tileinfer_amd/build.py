@@ -1,8 +1,9 @@
-"""Builds libtileinfer_amd.so (the gfx950 kernels + C ABI) in-tree with hipcc.
+"""Builds libtileinfer_amd.so (the gfx950 kernels + C ABI) in-tree with hipcc, and _pycalls.so (the
+Python entry points' common form in native code, csrc/pycalls.cpp) with the host compiler.
 
-Usage: ``python -m tileinfer_amd.build`` (or ``tileinfer_amd.build.build()``). The library lands
-next to this file, where :mod:`tileinfer_amd._lib` loads it; object files go to ``_build/``.
-Cross-compiles on a host without a GPU.
+Usage: ``python -m tileinfer_amd.build`` (or ``tileinfer_amd.build.build()``). Both land next to this
+file, where :mod:`tileinfer_amd._lib` loads them; object files go to ``_build/``. Cross-compiles on a
+host without a GPU.
 """
 from __future__ import annotations
 
@@ -11,6 +12,7 @@ import os
 import shutil
 import subprocess
 import sys
+import sysconfig
 from pathlib import Path
 
 PKG_DIR = Path(__file__).resolve().parent
@@ -18,6 +20,7 @@ CSRC = PKG_DIR / "csrc"
 BUILD_DIR = PKG_DIR / "_build"
 LIB_NAME = "libtileinfer_amd.so"
 LIB_PATH = PKG_DIR / LIB_NAME
+CALLS_PATH = PKG_DIR / "_pycalls.so"
 
 ARCH = os.environ.get("TI_OFFLOAD_ARCH", "gfx950")
 
@@ -59,14 +62,40 @@ def _compile(hipcc: str, src: Path, extra: list[str]) -> Path:
     return obj
 
 
+def _build_calls() -> None:
+    """csrc/pycalls.cpp against torch's headers (host code only)."""
+    import torch
+    from torch.utils import cpp_extension
+
+    cxx = os.environ.get("CXX") or shutil.which("g++") or shutil.which("clang++")
+    if cxx is None:
+        raise RuntimeError("no C++ compiler found for pycalls.cpp (set CXX)")
+    tmp = CALLS_PATH.with_suffix(".so.tmp")
+    lib_dir = Path(torch.__file__).resolve().parent / "lib"
+    cmd = [cxx, "-O2", "-std=c++17", "-fPIC", "-shared", "-Wall",
+           f"-D_GLIBCXX_USE_CXX11_ABI={int(torch._C._GLIBCXX_USE_CXX11_ABI)}",
+           *(f"-isystem{p}" for p in cpp_extension.include_paths()),
+           f"-isystem{sysconfig.get_paths()['include']}", str(CSRC / "pycalls.cpp"), "-o", str(tmp),
+           f"-L{lib_dir}", "-ltorch_python", "-ltorch_cpu", "-lc10"]
+    res = subprocess.run(cmd, capture_output=True, text=True)
+    if res.returncode != 0:
+        raise RuntimeError(f"host compiler failed on pycalls.cpp:\n{' '.join(cmd)}\n{res.stderr}")
+    if res.stderr.strip():
+        print(res.stderr, file=sys.stderr)
+    os.replace(tmp, CALLS_PATH)
+
+
 def build(verbose: bool = True, extra_flags: list[str] | None = None) -> Path:
-    """Compile every csrc/*.hip for gfx950 and link libtileinfer_amd.so. Always rebuilds."""
+    """Compile every csrc/*.hip for gfx950 and link libtileinfer_amd.so, and compile _pycalls.so.
+    Always rebuilds."""
     hipcc = _hipcc()
     BUILD_DIR.mkdir(exist_ok=True)
     extra = list(extra_flags or [])
     srcs = sources()
-    with cf.ThreadPoolExecutor(max_workers=min(8, len(srcs))) as ex:
+    with cf.ThreadPoolExecutor(max_workers=min(8, len(srcs) + 1)) as ex:
+        calls = ex.submit(_build_calls)
         objs = list(ex.map(lambda s: _compile(hipcc, s, extra), srcs))
+        calls.result()
     tmp = LIB_PATH.with_suffix(".so.tmp")
     cmd = [hipcc, f"--offload-arch={ARCH}", "-shared", "-fPIC", *map(str, objs), "-o", str(tmp)]
     res = subprocess.run(cmd, capture_output=True, text=True)

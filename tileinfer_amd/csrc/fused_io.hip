@@ -21,6 +21,25 @@
 namespace ti {
 namespace {
 
+// x rounded to 32 bits. Without this the compiler may fold the last operation before a conversion to
+// fp16 into it (one rounding instead of two), in one kernel and not in another; the forms below have
+// to give the same bits.
+__device__ __forceinline__ float rounded(float x) {
+  asm("" : "+v"(x));
+  return x;
+}
+
+// One rotated value: the first half of the pair (low) or the second.
+__device__ __forceinline__ float rotate(float own, float partner, float c, float s, bool low) {
+  const float ps = rounded(partner * s);
+  return rounded(fmaf(own, c, low ? -ps : ps));
+}
+
+// One normalised value: v times the row's scale r and the weight's 1 + w.
+__device__ __forceinline__ float normed(float v, float r, float w) {
+  return rounded(rounded(v * r) * (1.f + w));
+}
+
 struct NormRopeArgs {
   const uint16_t* x;
   int64_t x_st, x_sh;
@@ -39,10 +58,6 @@ struct NormRopeArgs {
   int64_t num_slots;
 };
 
-// One rotated value: the first half of the pair (low) or the second.
-__device__ __forceinline__ float rotate(float own, float partner, float c, float s, bool low) {
-  return fmaf(own, c, low ? -(partner * s) : partner * s);
-}
 
 // Rows of 16-byte aligned vectors (every stride a multiple of 8 elements, rotary_dim of 16): a row is
 // D / 8 lanes of 8 elements, so a wave takes 2 (D = 256) or 4 (D = 128) rows at once, and a
@@ -97,7 +112,7 @@ __device__ __forceinline__ u32x4 norm_rope_vec(const NormRopeArgs& a, u32x4 x, u
 #pragma unroll
   for (int j = 0; j < 4; ++j) {
     const float2 q = unpack2(w[j], Tag{});
-    nb[j] = pack2(v[2 * j] * r * (1.f + q.x), v[2 * j + 1] * r * (1.f + q.y), Tag{});
+    nb[j] = pack2(normed(v[2 * j], r, q.x), normed(v[2 * j + 1], r, q.y), Tag{});
   }
   if (a.rotary_dim == 0) return nb;  // uniform
   const int half = a.rotary_dim / 2;
@@ -192,7 +207,7 @@ __device__ __forceinline__ void norm_rope_row(const NormRopeArgs& a, int t, int 
   uint32_t nb[EPL / 2];
 #pragma unroll
   for (int j = 0; j < EPL; j += 2) {
-    nb[j / 2] = pack2(v[j] * r * (1.f + w[j]), v[j + 1] * r * (1.f + w[j + 1]), Tag{});
+    nb[j / 2] = pack2(normed(v[j], r, w[j]), normed(v[j + 1], r, w[j + 1]), Tag{});
     *reinterpret_cast<uint32_t*>(sh + EPL * lane + j) = nb[j / 2];
   }
   __builtin_amdgcn_wave_barrier();

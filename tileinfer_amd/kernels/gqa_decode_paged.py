@@ -227,6 +227,17 @@ def gqa_decode_paged_fn(
     Returns:
         [B, H_q, D] tensor in q's dtype.
     """
+    # The call in its common form (operands used as they are, the library's own choices) is checked
+    # and made in native code; None: another form, or one to refuse.
+    if (out is None and split_tokens is None and kv_reuse is None and not shared_prefix_tokens
+            and variant == "auto" and type(q) is torch.Tensor and q.is_cuda
+            and (append is None or (type(append) is tuple and len(append) == 3))):
+        key, value, slots = append or (None, None, None)
+        r = _lib.result(_lib.calls().decode(
+            q, k_cache, v_cache, block_table, seqlen_kv, page_size, gate, key, value, slots,
+            _lib.current_stream(q.get_device())))
+        if r is not None:
+            return r
     q, block_table, seqlen_kv, (b, h_q, d, h_kv, rows, page_size, dt, code, dev) = _checked(
         q, k_cache, v_cache, block_table, seqlen_kv, page_size, variant)
     if append is not None and (gate is not None or shared_prefix_tokens or variant == "scalar"):

@@ -140,6 +140,20 @@ def gqa_prefill_paged_fn(
     Returns:
         [total_q, H_q, D] tensor in q's dtype.
     """
+    # The call in its common form is checked and made in native code (see gqa_decode_paged_fn).
+    if (out is None and type(q) is torch.Tensor and q.is_cuda and q.dim() == 3 and q.shape[0]
+            and k_cache.dim() == 4 and k_cache.shape[2] > 0 and type(max_seqlen_q) is int
+            and type(causal) is bool and schedule in ("auto", "balanced", "per_unit")
+            and block_table.dim() == 2):
+        per_unit = bool(batch_invariant or schedule == "per_unit" or (
+            schedule == "auto" and _choose_per_unit(
+                block_table.shape[0], q.shape[0], max_seqlen_q, max_seqlen_k, causal, q.shape[1],
+                k_cache.shape[2], q.shape[2], q.device)))
+        r = _lib.result(_lib.calls().prefill(
+            q, k_cache, v_cache, block_table, cu_seqlens_q, seqlen_k, max_seqlen_q, page_size,
+            causal, per_unit, gate, _lib.current_stream(q.get_device())))
+        if r is not None:
+            return r
     if q.dim() != 3:
         raise ValueError(f"q must be [total_q, H_q, D], got {tuple(q.shape)}")
     total_q, h_q, d = q.shape

@@ -50,6 +50,11 @@ def store_kvcache(
         validate: keyword-only; also check on the host (synchronising) that every slot is in
             ``[-1, num_slots)`` and that non-negative slots are unique.
     """
+    # The call in its common form is checked and made in native code.
+    if (not validate and type(key) is torch.Tensor and key.is_cuda
+            and _lib.result(_lib.calls().append(key, value, k_cache, v_cache, slot_mapping,
+                                                _lib.current_stream(key.get_device()))) is True):
+        return
     if key.dim() != 3:
         raise ValueError(f"key must be [N, num_heads, head_dim], got {tuple(key.shape)}")
     n, num_heads, head_dim = key.shape

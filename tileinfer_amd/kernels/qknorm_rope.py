@@ -102,6 +102,13 @@ def qknorm_rope_append(q: torch.Tensor, k: torch.Tensor, v: torch.Tensor,
     ``[num_slots, H_kv * D]`` (the views ``store_kvcache`` takes); ``slot_mapping`` ``[T]`` int32
     (slots < 0 are skipped). K is written normalised and rotated, V as is.
     """
+    # The call in its common form is checked and made in native code.
+    if q_out is None and type(q) is torch.Tensor and q.is_cuda and type(eps) is float:
+        r = _lib.result(_lib.calls().qknorm_append(q, k, v, q_weight, k_weight, cos, sin, k_cache,
+                                                   v_cache, slot_mapping, eps,
+                                                   _lib.current_stream(q.get_device())))
+        if r is not None:
+            return r
     if q.dim() != 3 or k.dim() != 3 or v.dim() != 3:
         raise ValueError("q, k, v must be [T, heads, D]")
     t, hq, d = q.shape
