@@ -168,3 +168,20 @@ def test_checks_catch_planted_mistakes(mutant):
     np.testing.assert_allclose(_ref(step).float().numpy(), exact, atol=ATOL, rtol=RTOL)
     with pytest.raises(AssertionError):
         np.testing.assert_allclose(mutant(step).float().numpy(), exact, atol=ATOL, rtol=RTOL)
+
+
+def test_auto_schedule_from_host_bounds():
+    """The automatic schedule's choices that need no device: first chunks and batches of contexts up
+    to 1,024 tokens run one workgroup per unit, longer batches are balanced; without max_seqlen_k the
+    block table's tokens bound the contexts."""
+    from tileinfer_amd.kernels.gqa_prefill_paged import _choose_per_unit
+
+    def per_unit(batch, max_q, max_k, bound, causal=True):
+        return _choose_per_unit(batch, batch * max_q, max_q, max_k, bound, causal, 24, 4, 256, None)
+    assert per_unit(8, 300, 300, 4096) and per_unit(1, 300, 300, 4096)      # first chunks
+    assert per_unit(1, 64, None, 64) and not per_unit(1, 64, None, 80)      # table of the chunk alone
+    assert per_unit(2, 16, 1024, 4096) and not per_unit(2, 16, 1025, 4096)
+    assert per_unit(2, 16, None, 1024) and not per_unit(2, 16, None, 1040)
+    assert per_unit(2, 16, 5000, 512)                                       # the table holds no more
+    assert per_unit(2, 16, 512, 4096, causal=False)
+    assert not per_unit(2, 2000, 2000, 4096, causal=False)

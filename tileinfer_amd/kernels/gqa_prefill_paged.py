@@ -25,8 +25,9 @@ work (units may be cut between workgroups and merged in fp32 afterwards, in a fi
 launches), which removes the partial last round of a continuation chunk and spreads a few long
 units over the whole GPU. ``schedule="auto"`` (default) picks per call from host-known sizes: the
 per-unit schedule when no sequence has cached context (``max_seqlen_k <= max_seqlen_q``: causal
-first chunks pack well heaviest-first), a greedy estimate of both for a single sequence, the
-balanced schedule otherwise (and whenever ``max_seqlen_k`` is not given).
+first chunks pack well heaviest-first) and for batches of contexts of at most 1,024 tokens, a greedy
+estimate of both for a single sequence, the balanced schedule otherwise. Without ``max_seqlen_k`` the
+block table's width bounds the contexts.
 """
 from __future__ import annotations
 
@@ -79,13 +80,26 @@ def _per_unit_wins(q_len: int, kv_len: int, causal: bool, h_kv: int, group: int,
     return max(loads) <= sum(costs) / wgs + _BALANCE_OVERHEAD
 
 
-def _choose_per_unit(batch: int, total_q: int, max_q: int, max_k: int | None, causal: bool,
-                     h_q: int, h_kv: int, d: int, dev: torch.device) -> bool:
-    if max_k is None:
-        return False
-    if causal and max_k <= max_q:
+# Batches whose contexts are known to hold at most this many tokens take one workgroup per unit: a
+# unit is then a few key tiles, and the balanced schedule's plan and merge launches and its longer
+# pipeline fill cost more than its even shares save. Graph time per call, per unit / balanced, us:
+# 2 chunks of 4 tokens over 100 cached 7.8 / 25.2, over 600 21.6 / 32.1, over 1,000 32.5 / 33.8, over
+# 1,500 46.3 / 34.9; 40 chunks of 64 over 300 47 / 69, over 600 68 / 81; 8 of 300 over 600 75 / 87;
+# 40 of 300 over 600 331 / 319 (the one shape measured where the rule loses). One KV head of 256 and
+# 8 of 128 cross between 1,000 and 1,500 tokens too.
+_SHORT_CONTEXT = 1024
+
+
+def _choose_per_unit(batch: int, total_q: int, max_q: int, max_k: int | None, bound: int,
+                     causal: bool, h_q: int, h_kv: int, d: int, dev: torch.device) -> bool:
+    """Schedule of an "auto" call from host-known sizes; `bound`: tokens the block table can hold."""
+    if max_k is None and max_q * (h_q // h_kv) > 65535 * 128:
+        return False  # beyond the per-unit grid
+    if causal and (bound if max_k is None else max_k) <= max_q:
         return True  # no cached context: first chunks
     if batch != 1:
+        return (bound if max_k is None else min(max_k, bound)) <= _SHORT_CONTEXT
+    if max_k is None:
         return False
     rows = 128 if d == 256 else 256           # rows of a workgroup (the kernel's launch shape)
     wgs = torch.cuda.get_device_properties(dev).multi_processor_count
@@ -143,12 +157,13 @@ def gqa_prefill_paged_fn(
     # The call in its common form is checked and made in native code (see gqa_decode_paged_fn).
     if (out is None and type(q) is torch.Tensor and q.is_cuda and q.dim() == 3 and q.shape[0]
             and k_cache.dim() == 4 and k_cache.shape[2] > 0 and type(max_seqlen_q) is int
-            and type(causal) is bool and schedule in ("auto", "balanced", "per_unit")
-            and block_table.dim() == 2):
+            and type(causal) is bool and type(page_size) is int
+            and schedule in ("auto", "balanced", "per_unit") and block_table.dim() == 2):
         per_unit = bool(batch_invariant or schedule == "per_unit" or (
             schedule == "auto" and _choose_per_unit(
-                block_table.shape[0], q.shape[0], max_seqlen_q, max_seqlen_k, causal, q.shape[1],
-                k_cache.shape[2], q.shape[2], q.device)))
+                block_table.shape[0], q.shape[0], max_seqlen_q, max_seqlen_k,
+                block_table.shape[1] * page_size, causal, q.shape[1], k_cache.shape[2], q.shape[2],
+                q.device)))
         r = _lib.result(_lib.calls().prefill(
             q, k_cache, v_cache, block_table, cu_seqlens_q, seqlen_k, max_seqlen_q, page_size,
             causal, per_unit, gate, _lib.current_stream(q.get_device())))
@@ -225,8 +240,8 @@ def gqa_prefill_paged_fn(
     if schedule not in ("auto", "balanced", "per_unit"):
         raise ValueError(f"schedule must be 'auto', 'balanced' or 'per_unit', got {schedule!r}")
     per_unit = batch_invariant or schedule == "per_unit" or (
-        schedule == "auto" and _choose_per_unit(batch, total_q, max_seqlen_q, max_seqlen_k, causal,
-                                                h_q, h_kv, d, dev))
+        schedule == "auto" and _choose_per_unit(batch, total_q, max_seqlen_q, max_seqlen_k,
+                                                width * page_size, causal, h_q, h_kv, d, dev))
     ws, ws_bytes = None, 0
     if not per_unit:
         ws_bytes = _workspace_bytes(batch, total_q, h_q, h_kv, d, page_size, width)
