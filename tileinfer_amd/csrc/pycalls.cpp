@@ -130,6 +130,19 @@ at::Tensor bytes_on(const at::Tensor& like, int64_t n) {
 
 void* stream_of(PyObject* o) { return PyLong_AsVoidPtr(o); }
 
+// Lets other Python threads run while the library call and the allocations before it do (an
+// allocation may wait for the GPU, a launch for room in its queue). Restored on every way out.
+class Unlocked {
+ public:
+  Unlocked() : state_(PyEval_SaveThread()) {}
+  ~Unlocked() { PyEval_RestoreThread(state_); }
+  Unlocked(const Unlocked&) = delete;
+  Unlocked& operator=(const Unlocked&) = delete;
+
+ private:
+  PyThreadState* state_;
+};
+
 PyObject* guarded(PyObject* (*f)(PyObject* const*), PyObject* const* a, Py_ssize_t n, Py_ssize_t want) {
   if (n != want) {
     PyErr_Format(PyExc_TypeError, "expected %zd arguments, got %zd", want, n);
@@ -165,33 +178,39 @@ PyObject* decode(PyObject* const* a) {
       }
     }
   }
-  int32_t split = 0, splits = 0;
-  int64_t ws_bytes = 0;
-  int rc = p_plan(int32_t(p.batch), int32_t(p.hq), int32_t(p.hkv), int32_t(p.d), int32_t(p.page),
-                  int32_t(p.width), 0, &split, &splits, &ws_bytes);
-  if (rc != TI_OK) return PyLong_FromLong(rc);
-  at::Tensor out = at::empty({p.batch, p.hq, p.d}, p.q->options());
-  at::Tensor ws;
-  if (ws_bytes > 0) ws = bytes_on(*p.q, ws_bytes);
-  void* wp = ws_bytes > 0 ? ws.data_ptr() : nullptr;
   void* stream = stream_of(a[10]);
-  const int32_t* table = static_cast<const int32_t*>(p.table->data_ptr());
-  const int32_t* lens = static_cast<const int32_t*>(seqlen->data_ptr());
+  at::Tensor out;
+  int rc;
+  {
+    Unlocked unlocked;
+    int32_t split = 0, splits = 0;
+    int64_t ws_bytes = 0;
+    rc = p_plan(int32_t(p.batch), int32_t(p.hq), int32_t(p.hkv), int32_t(p.d), int32_t(p.page),
+                int32_t(p.width), 0, &split, &splits, &ws_bytes);
+    if (rc == TI_OK) {
+      out = at::empty({p.batch, p.hq, p.d}, p.q->options());
+      at::Tensor ws;
+      if (ws_bytes > 0) ws = bytes_on(*p.q, ws_bytes);
+      void* wp = ws_bytes > 0 ? ws.data_ptr() : nullptr;
+      const int32_t* table = static_cast<const int32_t*>(p.table->data_ptr());
+      const int32_t* lens = static_cast<const int32_t*>(seqlen->data_ptr());
 #define TI_DECODE_ARGS                                                                            \
   p.q->data_ptr(), p.q->stride(0), p.q->stride(1), p.k->data_ptr(), p.v->data_ptr(), table,       \
       p.table->stride(0), lens, out.data_ptr(), wp, ws_bytes, int32_t(p.batch), int32_t(p.hq),    \
       int32_t(p.hkv), int32_t(p.d), int32_t(p.page), p.rows / p.page, int32_t(p.width), 0,        \
       TI_DECODE_AUTO, p.dtype
-  if (key) {
-    rc = p_decode_append(TI_DECODE_ARGS, key->data_ptr(), value->data_ptr(), key->stride(0),
-                         value->stride(0), static_cast<const int32_t*>(slots->data_ptr()), p.rows,
-                         stream);
-  } else if (gate) {
-    rc = p_decode_gated(TI_DECODE_ARGS, gate->data_ptr(), p.hq * p.d, p.d, stream);
-  } else {
-    rc = p_decode(TI_DECODE_ARGS, stream);
-  }
+      if (key) {
+        rc = p_decode_append(TI_DECODE_ARGS, key->data_ptr(), value->data_ptr(), key->stride(0),
+                             value->stride(0), static_cast<const int32_t*>(slots->data_ptr()),
+                             p.rows, stream);
+      } else if (gate) {
+        rc = p_decode_gated(TI_DECODE_ARGS, gate->data_ptr(), p.hq * p.d, p.d, stream);
+      } else {
+        rc = p_decode(TI_DECODE_ARGS, stream);
+      }
 #undef TI_DECODE_ARGS
+    }
+  }
   if (rc != TI_OK) return PyLong_FromLong(rc);
   return THPVariable_Wrap(std::move(out));
 }
@@ -211,16 +230,21 @@ PyObject* prefill(PyObject* const* a) {
     Py_RETURN_NONE;
   }
   const bool causal = a[8] == Py_True, per_unit = a[9] == Py_True;
-  int64_t ws_bytes = 0;
-  if (!per_unit) {
-    const int rc = p_prefill_ws(int32_t(p.batch), int32_t(p.rows_q), int32_t(p.hq), int32_t(p.hkv),
-                                int32_t(p.d), int32_t(p.page), int32_t(p.width), &ws_bytes);
-    if (rc != TI_OK) return PyLong_FromLong(rc);
-  }
-  at::Tensor out = at::empty({p.rows_q, p.hq, p.d}, p.q->options());
-  at::Tensor ws;
-  if (ws_bytes > 0) ws = bytes_on(*p.q, ws_bytes);
-  void* wp = ws_bytes > 0 ? ws.data_ptr() : nullptr;
+  void* stream = stream_of(a[11]);
+  at::Tensor out;
+  int rc = TI_OK;
+  {
+    Unlocked unlocked;
+    int64_t ws_bytes = 0;
+    if (!per_unit) {
+      rc = p_prefill_ws(int32_t(p.batch), int32_t(p.rows_q), int32_t(p.hq), int32_t(p.hkv),
+                        int32_t(p.d), int32_t(p.page), int32_t(p.width), &ws_bytes);
+    }
+    if (rc == TI_OK) {
+      out = at::empty({p.rows_q, p.hq, p.d}, p.q->options());
+      at::Tensor ws;
+      if (ws_bytes > 0) ws = bytes_on(*p.q, ws_bytes);
+      void* wp = ws_bytes > 0 ? ws.data_ptr() : nullptr;
 #define TI_PREFILL_ARGS                                                                           \
   p.q->data_ptr(), p.q->stride(0), p.q->stride(1), p.k->data_ptr(), p.v->data_ptr(),              \
       static_cast<const int32_t*>(p.table->data_ptr()), p.table->stride(0),                       \
@@ -228,10 +252,11 @@ PyObject* prefill(PyObject* const* a) {
       out.data_ptr(), out.stride(0), out.stride(1), wp, ws_bytes, int32_t(p.batch),               \
       int32_t(p.rows_q), int32_t(max_q), int32_t(p.hq), int32_t(p.hkv), int32_t(p.d),             \
       int32_t(p.page), p.rows / p.page, int32_t(p.width), causal ? 1 : 0, p.dtype
-  const int rc = gate ? p_prefill_gated(TI_PREFILL_ARGS, gate->data_ptr(), p.hq * p.d, p.d,
-                                        stream_of(a[11]))
-                      : p_prefill(TI_PREFILL_ARGS, stream_of(a[11]));
+      rc = gate ? p_prefill_gated(TI_PREFILL_ARGS, gate->data_ptr(), p.hq * p.d, p.d, stream)
+                : p_prefill(TI_PREFILL_ARGS, stream);
 #undef TI_PREFILL_ARGS
+    }
+  }
   if (rc != TI_OK) return PyLong_FromLong(rc);
   return THPVariable_Wrap(std::move(out));
 }
@@ -261,10 +286,14 @@ PyObject* append(PyObject* const* a) {
   for (const at::Tensor* t : {key, value}) {
     if (t->stride(2) != 1 || t->stride(1) != d || t->stride(0) < h * d) Py_RETURN_NONE;
   }
-  const int rc = p_append(key->data_ptr(), value->data_ptr(), key->stride(0), value->stride(0),
-                          k->data_ptr(), v->data_ptr(), k->stride(0),
-                          static_cast<const int32_t*>(slots->data_ptr()), n, h * d, k->size(0), code,
-                          stream_of(a[5]));
+  void* stream = stream_of(a[5]);
+  int rc;
+  {
+    Unlocked unlocked;
+    rc = p_append(key->data_ptr(), value->data_ptr(), key->stride(0), value->stride(0),
+                  k->data_ptr(), v->data_ptr(), k->stride(0),
+                  static_cast<const int32_t*>(slots->data_ptr()), n, h * d, k->size(0), code, stream);
+  }
   if (rc != TI_OK) return PyLong_FromLong(rc);
   Py_RETURN_TRUE;
 }
@@ -302,14 +331,21 @@ PyObject* qknorm_append(PyObject* const* a) {
       !cache_rows(t[7], t[8], hkv * d, q) || !int32_vector(slots, n, q.device())) {
     Py_RETURN_NONE;
   }
-  at::Tensor out = at::empty({n, hq, d}, q.options());
-  const int rc = p_qknorm_append(
-      q.data_ptr(), q.stride(0), q.stride(1), k.data_ptr(), k.stride(0), k.stride(1), v.data_ptr(),
-      v.stride(0), v.stride(1), qw.data_ptr(), kw.data_ptr(), cos.data_ptr(), sin.data_ptr(),
-      n == 1 ? 0 : cos.stride(0), out.data_ptr(), out.stride(0), out.stride(1), t[7]->data_ptr(),
-      t[8]->data_ptr(), t[7]->stride(0), static_cast<const int32_t*>(slots.data_ptr()),
-      t[7]->size(0), int32_t(n), int32_t(hq), int32_t(hkv), int32_t(d), int32_t(rd),
-      float(PyFloat_AS_DOUBLE(a[10])), code, stream_of(a[11]));
+  const float eps = float(PyFloat_AS_DOUBLE(a[10]));
+  void* stream = stream_of(a[11]);
+  at::Tensor out;
+  int rc;
+  {
+    Unlocked unlocked;
+    out = at::empty({n, hq, d}, q.options());
+    rc = p_qknorm_append(
+        q.data_ptr(), q.stride(0), q.stride(1), k.data_ptr(), k.stride(0), k.stride(1), v.data_ptr(),
+        v.stride(0), v.stride(1), qw.data_ptr(), kw.data_ptr(), cos.data_ptr(), sin.data_ptr(),
+        n == 1 ? 0 : cos.stride(0), out.data_ptr(), out.stride(0), out.stride(1), t[7]->data_ptr(),
+        t[8]->data_ptr(), t[7]->stride(0), static_cast<const int32_t*>(slots.data_ptr()),
+        t[7]->size(0), int32_t(n), int32_t(hq), int32_t(hkv), int32_t(d), int32_t(rd), eps, code,
+        stream);
+  }
   if (rc != TI_OK) return PyLong_FromLong(rc);
   return THPVariable_Wrap(std::move(out));
 }
