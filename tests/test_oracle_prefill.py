@@ -185,3 +185,7 @@ def test_auto_schedule_from_host_bounds():
     assert per_unit(2, 16, 5000, 512)                                       # the table holds no more
     assert per_unit(2, 16, 512, 4096, causal=False)
     assert not per_unit(2, 2000, 2000, 4096, causal=False)
+    # A max_seqlen_q above the tokens, or beyond the per-unit grid, keeps the balanced schedule.
+    assert not _choose_per_unit(2, 32, 4096, None, 512, True, 24, 4, 256, None)
+    assert not _choose_per_unit(2, 32, 4096, 512, 512, False, 24, 4, 256, None)
+    assert not per_unit(2, 1 << 21, None, 1024) and not per_unit(2, 1 << 21, 1024, 1024, causal=False)

@@ -93,12 +93,15 @@ _SHORT_CONTEXT = 1024
 def _choose_per_unit(batch: int, total_q: int, max_q: int, max_k: int | None, bound: int,
                      causal: bool, h_q: int, h_kv: int, d: int, dev: torch.device) -> bool:
     """Schedule of an "auto" call from host-known sizes; `bound`: tokens the block table can hold."""
-    if max_k is None and max_q * (h_q // h_kv) > 65535 * 128:
-        return False  # beyond the per-unit grid
-    if causal and (bound if max_k is None else max_k) <= max_q:
+    if causal and max_k is not None and max_k <= max_q:
         return True  # no cached context: first chunks
+    # A max_seqlen_q above the call's tokens is no bound to size a grid by, and one workgroup per unit
+    # takes at most 65,535 row blocks of 128.
+    loose = max_q > total_q or max_q * (h_q // h_kv) > 65535 * 128
+    if causal and max_k is None and bound <= max_q and not loose:
+        return True  # the table holds no more than the chunks
     if batch != 1:
-        return (bound if max_k is None else min(max_k, bound)) <= _SHORT_CONTEXT
+        return not loose and (bound if max_k is None else min(max_k, bound)) <= _SHORT_CONTEXT
     if max_k is None:
         return False
     rows = 128 if d == 256 else 256           # rows of a workgroup (the kernel's launch shape)
