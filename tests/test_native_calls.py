@@ -110,6 +110,24 @@ def test_decode(which, form, dev, monkeypatch):
 
 
 @pytest.mark.gpu
+@pytest.mark.parametrize("gated", [False, True])
+@pytest.mark.parametrize("missing", [(0,), (1,), (2,), (0, 1, 2)])
+def test_append_without_an_operand_is_refused(missing, gated, dev, monkeypatch):
+    """An append= with None in it is no call without an append: it raises, and no cache row changes."""
+    say(f"native decode append without {missing} gated={gated}")
+    s = make_step([1, 17, 300], 64, seed=3)
+    q, k, v, table, lens, slots = (t.to(dev) for t in (s.q, s.k_cache, s.v_cache, s.block_table,
+                                                       s.seqlen, s.slot_mapping))
+    append = tuple(None if i in missing else t
+                   for i, t in enumerate((s.k_new.to(dev), s.v_new.to(dev), slots)))
+    gate = torch.zeros_like(q) if gated else None
+    before = k.clone(), v.clone()
+    assert both(monkeypatch, lambda: (gqa_decode_paged_fn(q, k, v, table, lens, s.page_size,
+                                                          gate=gate, append=append),)) is ValueError
+    assert torch.equal(bits(k), bits(before[0])) and torch.equal(bits(v), bits(before[1]))
+
+
+@pytest.mark.gpu
 @pytest.mark.parametrize("form", list(_FORMS))
 @pytest.mark.parametrize("which", ["q", "table", "lens", "gate"])
 @pytest.mark.parametrize("schedule", ["auto", "balanced"])

@@ -228,10 +228,12 @@ def gqa_decode_paged_fn(
         [B, H_q, D] tensor in q's dtype.
     """
     # The call in its common form (operands used as they are, the library's own choices) is checked
-    # and made in native code; None: another form, or one to refuse.
+    # and made in native code; None: another form, or one to refuse. (There a key of None says that
+    # no append is asked for, so an append without a key is refused below.)
     if (out is None and split_tokens is None and kv_reuse is None and not shared_prefix_tokens
             and variant == "auto" and type(q) is torch.Tensor and q.is_cuda
-            and (append is None or (type(append) is tuple and len(append) == 3))):
+            and (append is None or (type(append) is tuple and len(append) == 3
+                                    and append[0] is not None))):
         key, value, slots = append or (None, None, None)
         r = _lib.result(_lib.calls().decode(
             q, k_cache, v_cache, block_table, seqlen_kv, page_size, gate, key, value, slots,
