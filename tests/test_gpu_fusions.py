@@ -184,3 +184,26 @@ def test_fused_decode_step_graph_capture_replay(dev):
         torch.cuda.synchronize()
         assert torch.equal(bits(out_g), bits(eager)), f"replay {r}"
         assert torch.equal(bits(kc_g), bits(kc)) and torch.equal(bits(vc_g), bits(vc)), f"cache {r}"
+
+
+@pytest.mark.parametrize("d,hq,hkv", [(256, 24, 4), (128, 32, 8)])
+def test_gated_fp16_calls_round_as_the_separate_gate(d, hq, hkv, dev):
+    """In fp16 a product and its conversion may be one instruction or two, with other bits: the gated
+    decode (whole contexts, split ones, short ones) and the gated prefill (per unit, balanced, cut and
+    merged) give the bits of the plain call followed by the gate there too."""
+    say(f"gated fp16 d={d}")
+    g = torch.Generator().manual_seed(3)
+    for ctx, split in (([1, 17, 300, 40], None), ([5000, 3, 700], None), ([2500, 900], 256)):
+        s = make_step(ctx, 2048, seed=21, dtype=torch.float16, hq=hq, hkv=hkv, d=d)
+        args = [t.to(dev) for t in (s.q, s.k_cache, s.v_cache, s.block_table, s.seqlen)] + [s.page_size]
+        gate = (3 * torch.randn(s.q.shape, generator=g)).to(torch.float16).to(dev)
+        plain = gqa_decode_paged_fn(*args, split_tokens=split)
+        gated = gqa_decode_paged_fn(*args, split_tokens=split, gate=gate)
+        assert torch.equal(bits(gated), bits(fused_sigmoid_mul(plain, gate))), (ctx, split)
+    s = prefill_step([300, 1, 64], [1500, 400, 64], seed=22, dtype=torch.float16, hq=hq, hkv=hkv, d=d)
+    args = [t.to(dev) for t in (s.q, s.k_cache, s.v_cache, s.block_table, s.cu_seqlens_q, s.seqlen_k)]
+    gate = (3 * torch.randn(s.q.shape, generator=g)).to(torch.float16).to(dev)
+    for schedule in ("per_unit", "balanced"):
+        call = lambda **k: gqa_prefill_paged_fn(*args, s.max_seqlen_q, s.page_size,  # noqa: E731
+                                                schedule=schedule, **k)
+        assert torch.equal(bits(call(gate=gate)), bits(fused_sigmoid_mul(call(), gate))), schedule

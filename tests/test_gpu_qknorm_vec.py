@@ -20,7 +20,8 @@ def shifted(t):
     return out
 
 
-@pytest.mark.parametrize("d,dtype", [(256, torch.bfloat16), (128, torch.float16), (128, torch.bfloat16)])
+@pytest.mark.parametrize("d,dtype", [(256, torch.bfloat16), (256, torch.float16),
+                                     (128, torch.float16), (128, torch.bfloat16)])
 @pytest.mark.parametrize("t,hq,hkv,rd", [(1, 1, 1, 0), (1, 24, 4, 64), (3, 5, 1, 16), (7, 6, 2, 128),
                                          (65, 3, 3, 64), (2600, 8, 2, 64)])
 def test_vector_form_equals_general_form(t, hq, hkv, rd, d, dtype, dev):

@@ -51,6 +51,31 @@ __device__ __forceinline__ float2 unpack2(uint32_t v, F16) {
   return make_float2(float(h[0]), float(h[1]));
 }
 
+// Two results rounded to the storage type, the first in the low half: the products x0 y0 and x1 y1, or
+// the sums a0 b0 + c0 and a1 b1 + c1. To fp16 the compiler rounds a product once (v_fma_mixlo_f16) or
+// twice (to 32 bits, then to 16), as it sees fit where the call stands, so that kernels meant to give the
+// same bits differ in a value of 15,000 or so. Taken one by one, each is always rounded once.
+__device__ __forceinline__ uint32_t pack_apart2(_Float16 x, _Float16 y) {
+  asm("" : "+v"(x));
+  asm("" : "+v"(y));
+  const f16x2_t v = {x, y};
+  return __builtin_bit_cast(uint32_t, v);
+}
+__device__ __forceinline__ uint32_t pack_mul2(float x0, float y0, float x1, float y1, Bf16 tag) {
+  return pack2(x0 * y0, x1 * y1, tag);
+}
+__device__ __forceinline__ uint32_t pack_mul2(float x0, float y0, float x1, float y1, F16) {
+  return pack_apart2(static_cast<_Float16>(x0 * y0), static_cast<_Float16>(x1 * y1));
+}
+__device__ __forceinline__ uint32_t pack_fma2(float a0, float b0, float c0, float a1, float b1, float c1,
+                                              Bf16 tag) {
+  return pack2(fmaf(a0, b0, c0), fmaf(a1, b1, c1), tag);
+}
+__device__ __forceinline__ uint32_t pack_fma2(float a0, float b0, float c0, float a1, float b1, float c1,
+                                              F16) {
+  return pack_apart2(static_cast<_Float16>(fmaf(a0, b0, c0)), static_cast<_Float16>(fmaf(a1, b1, c1)));
+}
+
 // Logistic function 1 / (1 + 2^(-x log2 e)) on the exp2 and reciprocal units (1 ulp each; the scaled
 // argument's rounding adds |x| 2^-24): within 4e-6 relative for |x| <= 40, against the 2^-9 (bf16)
 // or 2^-11 (fp16) of the product it goes into. expf and an IEEE division take ~40 instructions
@@ -66,7 +91,7 @@ template <typename Tag>
 __device__ __forceinline__ uint32_t gate_mul2(uint32_t a, uint32_t g, Tag tag) {
   const float2 x = unpack2(a, tag);
   const float2 y = unpack2(g, tag);
-  return pack2(x.x * sigmoidf(y.x), x.y * sigmoidf(y.y), tag);
+  return pack_mul2(x.x, sigmoidf(y.x), x.y, sigmoidf(y.y), tag);
 }
 
 __device__ __forceinline__ u32x4 load16(const uint16_t* p) {

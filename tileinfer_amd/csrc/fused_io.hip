@@ -21,23 +21,18 @@
 namespace ti {
 namespace {
 
-// x rounded to 32 bits. Without this the compiler may fold the last operation before a conversion to
-// fp16 into it (one rounding instead of two), in one kernel and not in another; the forms below have
-// to give the same bits.
+// x rounded to 32 bits: the compiler may not fold it into what follows, in one kernel and not in
+// another; the forms below have to give the same bits.
 __device__ __forceinline__ float rounded(float x) {
   asm("" : "+v"(x));
   return x;
 }
 
-// One rotated value: the first half of the pair (low) or the second.
-__device__ __forceinline__ float rotate(float own, float partner, float c, float s, bool low) {
+// A rotated value is own * c + this: the partner's part in the first half of the pair (low) or the
+// second.
+__device__ __forceinline__ float partner_part(float partner, float s, bool low) {
   const float ps = rounded(partner * s);
-  return rounded(fmaf(own, c, low ? -ps : ps));
-}
-
-// One normalised value: v times the row's scale r and the weight's 1 + w.
-__device__ __forceinline__ float normed(float v, float r, float w) {
-  return rounded(rounded(v * r) * (1.f + w));
+  return low ? -ps : ps;
 }
 
 struct NormRopeArgs {
@@ -112,7 +107,7 @@ __device__ __forceinline__ u32x4 norm_rope_vec(const NormRopeArgs& a, u32x4 x, u
 #pragma unroll
   for (int j = 0; j < 4; ++j) {
     const float2 q = unpack2(w[j], Tag{});
-    nb[j] = pack2(normed(v[2 * j], r, q.x), normed(v[2 * j + 1], r, q.y), Tag{});
+    nb[j] = pack_mul2(rounded(v[2 * j] * r), 1.f + q.x, rounded(v[2 * j + 1] * r), 1.f + q.y, Tag{});
   }
   if (a.rotary_dim == 0) return nb;  // uniform
   const int half = a.rotary_dim / 2;
@@ -133,8 +128,8 @@ __device__ __forceinline__ u32x4 norm_rope_vec(const NormRopeArgs& a, u32x4 x, u
     const float2 partner = unpack2(pb[j], Tag{});
     const float2 cc = unpack2(c[j], Tag{});
     const float2 s2 = unpack2(sn[j], Tag{});
-    res[j] = pack2(rotate(own.x, partner.x, cc.x, s2.x, low), rotate(own.y, partner.y, cc.y, s2.y, low),
-                   Tag{});
+    res[j] = pack_fma2(own.x, cc.x, partner_part(partner.x, s2.x, low), own.y, cc.y,
+                       partner_part(partner.y, s2.y, low), Tag{});
   }
   return res;
 }
@@ -207,7 +202,7 @@ __device__ __forceinline__ void norm_rope_row(const NormRopeArgs& a, int t, int 
   uint32_t nb[EPL / 2];
 #pragma unroll
   for (int j = 0; j < EPL; j += 2) {
-    nb[j / 2] = pack2(normed(v[j], r, w[j]), normed(v[j + 1], r, w[j + 1]), Tag{});
+    nb[j / 2] = pack_mul2(rounded(v[j] * r), 1.f + w[j], rounded(v[j + 1] * r), 1.f + w[j + 1], Tag{});
     *reinterpret_cast<uint32_t*>(sh + EPL * lane + j) = nb[j / 2];
   }
   __builtin_amdgcn_wave_barrier();
@@ -219,7 +214,7 @@ __device__ __forceinline__ void norm_rope_row(const NormRopeArgs& a, int t, int 
 #pragma unroll
   for (int j = 0; j < EPL; j += 2) {
     const float2 own = unpack2(nb[j / 2], Tag{});
-    float o2[2] = {own.x, own.y};
+    float c2[2] = {1.f, 1.f}, p2[2] = {-0.f, -0.f};  // past the rotation: the value itself
 #pragma unroll
     for (int e = 0; e < 2; ++e) {
       const int i = EPL * lane + j + e;
@@ -228,12 +223,11 @@ __device__ __forceinline__ void norm_rope_row(const NormRopeArgs& a, int t, int 
         const int pi = i < half ? i + half : i - half;  // rotation partner
         const uint16_t pb = sh[pi];
         const float partner = unpack2(uint32_t(pb), Tag{}).x;
-        const float c = unpack2(uint32_t(cr[k]), Tag{}).x;
-        const float s = unpack2(uint32_t(sr[k]), Tag{}).x;
-        o2[e] = rotate(o2[e], partner, c, s, i < half);
+        c2[e] = unpack2(uint32_t(cr[k]), Tag{}).x;
+        p2[e] = partner_part(partner, unpack2(uint32_t(sr[k]), Tag{}).x, i < half);
       }
     }
-    res[j / 2] = pack2(o2[0], o2[1], Tag{});
+    res[j / 2] = pack_fma2(own.x, c2[0], p2[0], own.y, c2[1], p2[1], Tag{});
   }
 }
 

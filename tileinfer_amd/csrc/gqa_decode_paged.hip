@@ -545,7 +545,7 @@ __global__ __launch_bounds__(64 * WPB) void decode_mfma_kernel(DecodeArgs a, int
           u32x4 w;
 #pragma unroll
           for (int k = 0; k < 4; ++k) {
-            w[k] = pack2(o[8 * c + 2 * k][r] * inv, o[8 * c + 2 * k + 1][r] * inv, Tag{});
+            w[k] = pack_mul2(o[8 * c + 2 * k][r], inv, o[8 * c + 2 * k + 1][r], inv, Tag{});
           }
           put(128 * c + 32 * g + 8 * r, w);
         }
@@ -587,7 +587,7 @@ __global__ __launch_bounds__(64 * WPB) void decode_mfma_kernel(DecodeArgs a, int
         }
         u32x4 w;
 #pragma unroll
-        for (int k = 0; k < 4; ++k) w[k] = pack2(acc[2 * k] * inv, acc[2 * k + 1] * inv, Tag{});
+        for (int k = 0; k < 4; ++k) w[k] = pack_mul2(acc[2 * k], inv, acc[2 * k + 1], inv, Tag{});
         put(d, w);
       }
     }
@@ -665,7 +665,7 @@ __global__ __launch_bounds__(64 * WPB) void decode_mfma_kernel(DecodeArgs a, int
       }
       u32x4 v;
 #pragma unroll
-      for (int k = 0; k < 4; ++k) v[k] = pack2(acc[2 * k] * inv, acc[2 * k + 1] * inv, Tag{});
+      for (int k = 0; k < 4; ++k) v[k] = pack_mul2(acc[2 * k], inv, acc[2 * k + 1], inv, Tag{});
       const int d = 128 * c + 32 * g + 8 * r;
       if (grow) {
         const u32x4 gv = load16(grow + d);
@@ -913,7 +913,7 @@ __global__ __launch_bounds__(64 * W) void decode_merge_kernel(DecodeArgs a, int 
         inv = l > 0.f ? 1.f / l : 0.f;
       }
 #pragma unroll
-      for (int j = 0; j < PER; j += 2) put(j, pack2(e[j] * inv, e[j + 1] * inv, Tag{}));
+      for (int j = 0; j < PER; j += 2) put(j, pack_mul2(e[j], inv, e[j + 1], inv, Tag{}));
       return;
     }
     // Where the sequence's tiles start in the batch's tile order, and the batch's total, as the
@@ -1028,7 +1028,7 @@ __global__ __launch_bounds__(64 * W) void decode_merge_kernel(DecodeArgs a, int 
       }
       const float inv = l > 0.f ? 1.f / l : 0.f;
 #pragma unroll
-      for (int j = 0; j < PER; j += 2) put(j, pack2(acc[j] * inv, acc[j + 1] * inv, Tag{}));
+      for (int j = 0; j < PER; j += 2) put(j, pack_mul2(acc[j], inv, acc[j + 1], inv, Tag{}));
       return;
     }
   }
@@ -1131,7 +1131,7 @@ __global__ __launch_bounds__(64 * W) void decode_merge_kernel(DecodeArgs a, int 
   }
   const float inv = l > 0.f ? 1.f / l : 0.f;
 #pragma unroll
-  for (int j = 0; j < PER; j += 2) put(j, pack2(acc[j] * inv, acc[j + 1] * inv, Tag{}));
+  for (int j = 0; j < PER; j += 2) put(j, pack_mul2(acc[j], inv, acc[j + 1], inv, Tag{}));
 }
 
 template <int D, typename Tag, int WPB, bool SMALL>

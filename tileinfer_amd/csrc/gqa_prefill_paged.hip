@@ -960,8 +960,8 @@ __global__ __launch_bounds__(64 * W) void prefill_mfma_kernel(PrefillArgs a) {
 #pragma unroll
       for (int dt = 0; dt < NT; ++dt) {
         u32x2 w;
-        w[0] = pack2(o[c][dt][0] * inv, o[c][dt][1] * inv, Tag{});
-        w[1] = pack2(o[c][dt][2] * inv, o[c][dt][3] * inv, Tag{});
+        w[0] = pack_mul2(o[c][dt][0], inv, o[c][dt][1], inv, Tag{});
+        w[1] = pack_mul2(o[c][dt][2], inv, o[c][dt][3], inv, Tag{});
         if (grow) {  // uniform
           const u32x2 gv = *reinterpret_cast<const u32x2*>(grow + 16 * dt + 4 * g);
           w[0] = gate_mul2(w[0], gv[0], Tag{});
@@ -1483,8 +1483,8 @@ __global__ __launch_bounds__(128 * kPairs) void prefill_pair_kernel(PrefillArgs 
 #pragma unroll
       for (int dt = 0; dt < NT; ++dt) {
         u32x2 x;
-        x[0] = pack2(o[c][dt][0] * inv, o[c][dt][1] * inv, Tag{});
-        x[1] = pack2(o[c][dt][2] * inv, o[c][dt][3] * inv, Tag{});
+        x[0] = pack_mul2(o[c][dt][0], inv, o[c][dt][1], inv, Tag{});
+        x[1] = pack_mul2(o[c][dt][2], inv, o[c][dt][3], inv, Tag{});
         if (grow) {  // uniform
           const u32x2 gv = *reinterpret_cast<const u32x2*>(grow + 16 * dt + 4 * g);
           x[0] = gate_mul2(x[0], gv[0], Tag{});
@@ -1759,10 +1759,10 @@ __global__ __launch_bounds__(256) void prefill_merge_kernel(PrefillArgs a) {
     uint16_t* orow = a.out + int64_t(sx.q_start + qb0 + tok) * a.o_st +
                      int64_t(kvh * a.group + hh) * a.o_sh + d0;
     u32x4 w;
-    w[0] = pack2(acc[j][0][0] * inv, acc[j][0][1] * inv, Tag{});
-    w[1] = pack2(acc[j][0][2] * inv, acc[j][0][3] * inv, Tag{});
-    w[2] = pack2(acc[j][1][0] * inv, acc[j][1][1] * inv, Tag{});
-    w[3] = pack2(acc[j][1][2] * inv, acc[j][1][3] * inv, Tag{});
+    w[0] = pack_mul2(acc[j][0][0], inv, acc[j][0][1], inv, Tag{});
+    w[1] = pack_mul2(acc[j][0][2], inv, acc[j][0][3], inv, Tag{});
+    w[2] = pack_mul2(acc[j][1][0], inv, acc[j][1][1], inv, Tag{});
+    w[3] = pack_mul2(acc[j][1][2], inv, acc[j][1][3], inv, Tag{});
     if (a.gate) {
       const u32x4 gv = *reinterpret_cast<const u32x4*>(
           a.gate + int64_t(sx.q_start + qb0 + tok) * a.gate_st +
