@@ -9,17 +9,21 @@ import torch
 
 from helpers import ATOL, RTOL, bits, say
 from oracle.ref_torch import ref_gqa_prefill_paged
-from tileinfer_amd.kernels.gqa_prefill_paged import gqa_prefill_paged_fn
+from tileinfer_amd.kernels import fused_sigmoid_mul, gqa_prefill_paged_fn
 from tileinfer_amd.workloads import prefill_step
 
 pytestmark = pytest.mark.gpu
 
 
+def run(step, dev, causal=True, **kw):
+    return gqa_prefill_paged_fn(step.q.to(dev), step.k_cache.to(dev), step.v_cache.to(dev),
+                                step.block_table.to(dev), step.cu_seqlens_q.to(dev),
+                                step.seqlen_k.to(dev), step.max_seqlen_q, step.page_size,
+                                causal=causal, schedule="balanced", **kw)
+
+
 def both(step, dev, causal=True):
-    out = gqa_prefill_paged_fn(step.q.to(dev), step.k_cache.to(dev), step.v_cache.to(dev),
-                               step.block_table.to(dev), step.cu_seqlens_q.to(dev),
-                               step.seqlen_k.to(dev), step.max_seqlen_q, step.page_size,
-                               causal=causal, schedule="balanced")
+    out = run(step, dev, causal)
     ref = ref_gqa_prefill_paged(step.q, step.k_cache, step.v_cache, step.block_table,
                                 step.cu_seqlens_q, step.seqlen_k, step.page_size, causal)
     return out, ref
@@ -38,6 +42,26 @@ def test_pipeline_edges_vs_oracle(q_lens, kv_lens, hq, hkv, dev):
     for causal in (True, False):
         out, ref = both(step, dev, causal)
         torch.testing.assert_close(out.float().cpu(), ref.float(), atol=ATOL, rtol=RTOL)
+
+
+@pytest.mark.parametrize("dtype", [torch.bfloat16, torch.float16])
+@pytest.mark.parametrize("q_lens,kv_lens", [
+    ([1], [1]), ([33], [33]), ([1] * 70, [1] * 70), ([3, 1, 40, 0, 5], [3, 33, 129, 7, 0]),
+    ([200, 31, 64], [700, 31, 900]),             # cut units: gated by the merge
+])
+def test_gate_is_applied_to_the_rounded_rows(q_lens, kv_lens, dtype, dev):
+    """The gated call gives the bits of the plain call followed by the gate, for gate rows of their
+    own and for rows that lie a stride apart, and changes no row of its operands."""
+    say(f"prefill pairs gated q={q_lens} kv={kv_lens} {dtype}")
+    step = prefill_step(q_lens, kv_lens, seed=53, dtype=dtype)
+    plain = run(step, dev)
+    gate = 3 * torch.randn(plain.shape, generator=torch.Generator().manual_seed(5))
+    gate = gate.to(dtype).to(dev)
+    apart = torch.empty(gate.shape[0], 2, *gate.shape[1:], dtype=dtype, device=dev)[:, 1].copy_(gate)
+    want = fused_sigmoid_mul(plain, gate)
+    for g in (gate, apart):
+        assert torch.equal(bits(run(step, dev, gate=g)), bits(want))
+    assert torch.equal(bits(apart), bits(gate))
 
 
 def test_values_outside_every_mask_stay_out(dev):

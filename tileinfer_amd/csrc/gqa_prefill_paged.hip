@@ -466,6 +466,46 @@ __device__ __forceinline__ SeqExtent walk_extent(const Walk& w) {
   return s;
 }
 
+// Stores output row (token tk, query head h): o times inv, and times the sigmoid of its gate where the
+// call has one. Lane (n, g) of the row's four holds d = 16 dt + 4g .. +3 in o[dt].
+// The branch is on a kernel argument (uniform) and the gate's vectors are requested eight d-tiles ahead
+// (16 registers, which is what an output wave of the pairs has left). Branching on the row's own
+// pointer made a divergent branch of every d-tile, each with a wait for its load and for all accesses
+// before it, a wave pair's K/V loads for the next tiles among them: 16 round trips per column tile.
+// Balanced, 24 chunks of 16 to 330 tokens over up to 2,000 cached: 243 -> 208 us (24/4 heads of 256),
+// 132 -> 111 (12/2); 40 of 100 to 330: 446 -> 378; per unit, 48 first chunks of 30 to 600: 261 -> 245.
+template <int NT, typename Tag>
+__device__ __forceinline__ void store_row(const PrefillArgs& a, const f32x4 (&o)[NT], float inv, int tk,
+                                          int h, int g, Tag tag) {
+  uint16_t* orow = a.out + int64_t(tk) * a.o_st + int64_t(h) * a.o_sh + 4 * g;
+  auto values = [&](int dt) __attribute__((always_inline)) {
+    return u32x2{pack_mul2(o[dt][0], inv, o[dt][1], inv, tag),
+                 pack_mul2(o[dt][2], inv, o[dt][3], inv, tag)};
+  };
+  if (a.gate == nullptr) {  // uniform
+#pragma unroll
+    for (int dt = 0; dt < NT; ++dt) *reinterpret_cast<u32x2*>(orow + 16 * dt) = values(dt);
+    return;
+  }
+  const uint16_t* grow = a.gate + int64_t(tk) * a.gate_st + int64_t(h) * a.gate_sh + 4 * g;
+  auto gate = [&](int dt) __attribute__((always_inline)) {
+    return *reinterpret_cast<const u32x2*>(grow + 16 * dt);
+  };
+  constexpr int R = 8;
+  u32x2 gv[R];
+#pragma unroll
+  for (int dt = 0; dt < R; ++dt) gv[dt] = gate(dt);
+#pragma unroll
+  for (int dt = 0; dt < NT; ++dt) {
+    __builtin_amdgcn_sched_barrier(0);
+    u32x2 x = values(dt);
+    x[0] = gate_mul2(x[0], gv[dt % R][0], tag);
+    x[1] = gate_mul2(x[1], gv[dt % R][1], tag);
+    if (dt + R < NT) gv[dt % R] = gate(dt + R);
+    *reinterpret_cast<u32x2*>(orow + 16 * dt) = x;
+  }
+}
+
 // A workgroup's rows are the (token, query head) pairs of one KV head's group, row = token * group
 // + head-in-group, 16 * C * W rows over W waves (C column tiles of 16 rows per wave). Every staged
 // K/V tile is thus shared by all query heads of the group, and every K/V operand read from LDS feeds
@@ -950,25 +990,8 @@ __global__ __launch_bounds__(64 * W) void prefill_mfma_kernel(PrefillArgs a) {
         }
         continue;
       }
-      uint16_t* orow =
-          a.out + int64_t(sx.q_start + tok) * a.o_st + int64_t(kvh * G + hh) * a.o_sh;
-      const float inv = l_tot > 0.f ? 1.f / l_tot : 0.f;
-      // Lane (n, g) holds d = 16 dt + 4g .. +3 of its row in o[c][dt].
-      const uint16_t* grow = a.gate ? a.gate + int64_t(sx.q_start + tok) * a.gate_st +
-                                          int64_t(kvh * G + hh) * a.gate_sh
-                                    : nullptr;
-#pragma unroll
-      for (int dt = 0; dt < NT; ++dt) {
-        u32x2 w;
-        w[0] = pack_mul2(o[c][dt][0], inv, o[c][dt][1], inv, Tag{});
-        w[1] = pack_mul2(o[c][dt][2], inv, o[c][dt][3], inv, Tag{});
-        if (grow) {  // uniform
-          const u32x2 gv = *reinterpret_cast<const u32x2*>(grow + 16 * dt + 4 * g);
-          w[0] = gate_mul2(w[0], gv[0], Tag{});
-          w[1] = gate_mul2(w[1], gv[1], Tag{});
-        }
-        *reinterpret_cast<u32x2*>(orow + 16 * dt + 4 * g) = w;
-      }
+      store_row<NT>(a, o[c], l_tot > 0.f ? 1.f / l_tot : 0.f, sx.q_start + tok, kvh * G + hh, g,
+                    Tag{});
     }
   };
 
@@ -1474,24 +1497,7 @@ __global__ __launch_bounds__(128 * kPairs) void prefill_pair_kernel(PrefillArgs 
         }
         continue;
       }
-      uint16_t* orow = a.out + int64_t(sx.q_start + tok) * a.o_st + int64_t(hh) * a.o_sh;
-      const float inv = l[c] > 0.f ? 1.f / l[c] : 0.f;
-      // Lane (n, g) holds d = 16 dt + 4g .. +3 of its row in o[c][dt].
-      const uint16_t* grow = a.gate ? a.gate + int64_t(sx.q_start + tok) * a.gate_st +
-                                          int64_t(hh) * a.gate_sh
-                                    : nullptr;
-#pragma unroll
-      for (int dt = 0; dt < NT; ++dt) {
-        u32x2 x;
-        x[0] = pack_mul2(o[c][dt][0], inv, o[c][dt][1], inv, Tag{});
-        x[1] = pack_mul2(o[c][dt][2], inv, o[c][dt][3], inv, Tag{});
-        if (grow) {  // uniform
-          const u32x2 gv = *reinterpret_cast<const u32x2*>(grow + 16 * dt + 4 * g);
-          x[0] = gate_mul2(x[0], gv[0], Tag{});
-          x[1] = gate_mul2(x[1], gv[1], Tag{});
-        }
-        *reinterpret_cast<u32x2*>(orow + 16 * dt + 4 * g) = x;
-      }
+      store_row<NT>(a, o[c], l[c] > 0.f ? 1.f / l[c] : 0.f, sx.q_start + tok, hh, g, Tag{});
     }
   };
   // V^T operand addresses for the transposed reads: lane (s, g) (s = lane % 16) points at key row
