@@ -207,3 +207,26 @@ def test_gated_fp16_calls_round_as_the_separate_gate(d, hq, hkv, dev):
         call = lambda **k: gqa_prefill_paged_fn(*args, s.max_seqlen_q, s.page_size,  # noqa: E731
                                                 schedule=schedule, **k)
         assert torch.equal(bits(call(gate=gate)), bits(fused_sigmoid_mul(call(), gate))), schedule
+
+
+@pytest.mark.parametrize("dtype", [torch.bfloat16, torch.float16])
+def test_gate_over_every_16_bit_value(dtype, dev):
+    """Every gate there is, NaN and infinities among them, times values of several sizes, against the
+    product in 64 bits. The factor's error is bounded by the exp2 unit's 1 ulp (2^-23), and half an ulp
+    each of its argument, the sum 1 + e, the reciprocal and the product: 3.5 * 2^-24 * 2 in all, so the
+    stored value is what the exact product rounds to when it is moved by at most that."""
+    say(f"gate, every {dtype} value")
+    gate = torch.arange(-32768, 32768, dtype=torch.int32).to(torch.int16).view(dtype)
+    worst = 3.5 * 2.0 ** -23
+    for a in (1.0, -1.39, 300.0, 3e4):
+        x = torch.full_like(gate, a)
+        out = fused_sigmoid_mul(x.to(dev), gate.to(dev)).cpu()
+        exact = x.double() * torch.sigmoid(gate.double())
+        # Below 2^-126 the factor itself is a rounded subnormal number: 2^-149 more either way.
+        near = torch.stack([exact * (1 - worst), exact * (1 + worst)])
+        lo = (near.amin(0) - abs(a) * 2.0 ** -149).to(dtype)
+        hi = (near.amax(0) + abs(a) * 2.0 ** -149).to(dtype)
+        nan = gate.isnan()
+        assert out[nan].isnan().all() and not out[~nan].isnan().any()
+        ok = (out >= lo) & (out <= hi)
+        assert ok[~nan].all(), (a, gate[~nan & ~ok][:8].tolist())
