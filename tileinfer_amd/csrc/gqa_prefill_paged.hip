@@ -472,8 +472,8 @@ __device__ __forceinline__ SeqExtent walk_extent(const Walk& w) {
 // (16 registers, which is what an output wave of the pairs has left). Branching on the row's own
 // pointer made a divergent branch of every d-tile, each with a wait for its load and for all accesses
 // before it, a wave pair's K/V loads for the next tiles among them: 16 round trips per column tile.
-// Balanced, 24 chunks of 16 to 330 tokens over up to 2,000 cached: 243 -> 208 us (24/4 heads of 256),
-// 132 -> 111 (12/2); 40 of 100 to 330: 446 -> 378; per unit, 48 first chunks of 30 to 600: 261 -> 245.
+// Balanced, 24 chunks of 16 to 330 tokens over up to 2,000 cached: 241 -> 203 us (24/4 heads of 256),
+// 130 -> 113 (12/2); 40 of 100 to 330: 447 -> 379; per unit, 48 first chunks of 30 to 600: 261 -> 250.
 template <int NT, typename Tag>
 __device__ __forceinline__ void store_row(const PrefillArgs& a, const f32x4 (&o)[NT], float inv, int tk,
                                           int h, int g, Tag tag) {
@@ -1464,14 +1464,15 @@ __global__ __launch_bounds__(128 * kPairs) void prefill_pair_kernel(PrefillArgs 
   clear();
   // Stores the piece's rows, given each row's (m, l): normalised into `out` (a whole unit), or
   // unnormalised (o relative to 2^m) into `uo` or the workgroup's partial slot.
-  auto store = [&](const float (&m)[C], const float (&l)[C]) __attribute__((always_inline)) {
+  auto store = [&](const float (&m)[C], const float (&l)[C], int rn, int rg)
+      __attribute__((always_inline)) {
     const SeqExtent sx = extent();
     const int ur = unit_rows(sx);
     const int qr0 = uni(w.qr0);
     const bool whole = uni(w.whole) != 0;
 #pragma unroll
     for (int c = 0; c < C; ++c) {
-      const int rho = pair * 16 * C + 16 * c + n;
+      const int rho = pair * 16 * C + 16 * c + rn;
       if (rho >= ur) continue;
       const int tok = (qr0 + rho) / G;
       const int hh = uni(w.kvh) * G + (qr0 + rho - tok * G);
@@ -1489,15 +1490,15 @@ __global__ __launch_bounds__(128 * kPairs) void prefill_pair_kernel(PrefillArgs 
         }
 #pragma unroll
         for (int dt = 0; dt < NT; ++dt) {
-          *reinterpret_cast<f32x4*>(po + 16 * dt + 4 * g) = o[c][dt];
+          *reinterpret_cast<f32x4*>(po + 16 * dt + 4 * rg) = o[c][dt];
         }
-        if (g == 0) {
+        if (rg == 0) {
           pml[0] = m[c];
           pml[1] = l[c];
         }
         continue;
       }
-      store_row<NT>(a, o[c], l[c] > 0.f ? 1.f / l[c] : 0.f, sx.q_start + tok, hh, g, Tag{});
+      store_row<NT>(a, o[c], l[c] > 0.f ? 1.f / l[c] : 0.f, sx.q_start + tok, hh, rg, Tag{});
     }
   };
   // V^T operand addresses for the transposed reads: lane (s, g) (s = lane % 16) points at key row
@@ -1652,13 +1653,19 @@ __global__ __launch_bounds__(128 * kPairs) void prefill_pair_kernel(PrefillArgs 
       ++done;
       stage = stage == kVStages - 1 ? 0 : stage + 1;
     }
+    // The lane's indices anew: what is formed from n and g here would otherwise be kept, spilled, across
+    // the pieces, and a spilled value's reload waits for the K/V loads in flight.
+    int rn;
+    asm volatile("v_mbcnt_lo_u32_b32 %0, -1, 0\n\tv_mbcnt_hi_u32_b32 %0, -1, %0" : "=v"(rn));
+    const int rg = rn >> 4;
+    rn &= 15;
     float m[C], l[C];
 #pragma unroll
     for (int c = 0; c < C; ++c) {
-      m[c] = s_ml[(done - 1) & 1][pair][c][0][n];
-      l[c] = s_ml[(done - 1) & 1][pair][c][1][n];
+      m[c] = s_ml[(done - 1) & 1][pair][c][0][rn];
+      l[c] = s_ml[(done - 1) & 1][pair][c][1][rn];
     }
-    store(m, l);
+    store(m, l, rn, rg);
     if (uni(w.fin) != 0 || !walk_next(a, w)) break;
     clear();
   }
