@@ -1861,8 +1861,16 @@ int launch_prefill(const PrefillArgs& a, int batch, int max_q, hipStream_t s) {
                     : a.page_shift >= 0 ? prefill_kernel<D, BAL, true, Tag>()
                                         : prefill_kernel<D, BAL, false, Tag>();
   if constexpr (!BAL) {
-    const dim3 grid(unsigned(a.hkv), unsigned(ceil_div(int64_t(max_q) * a.group, S::ROWS)),
-                    unsigned(batch * a.key_splits));
+    unsigned blocks = unsigned(ceil_div(int64_t(max_q) * a.group, S::ROWS));
+    // Workgroup ids go round-robin over the 8 XCDs and, as the times below show, over 4 groups of CUs in
+    // each. With an even number of blocks per sequence (a power of two above all) the first blocks of
+    // the sequences, which are all that short ones have, land on some of the 32 only; an odd one spreads
+    // them (at the price of a block without rows per sequence and KV head, ~5 ns). 4
+    // chunks of 200 over 600 and 60 of 16 over 384, 32/8 heads of 128 (4 blocks): 143 -> 62 us, 24/4 of
+    // 256 (10): 67 -> 50; a chunk of 150 and 255 of one token, 24/4 (8): 582 -> 132. Batches of one length
+    // gain from the changed order or stay: 16 first chunks of 512 111 -> 103, 8 of 2,048 509 -> 507.
+    if (batch > 1) blocks |= 1;
+    const dim3 grid(unsigned(a.hkv), blocks, unsigned(batch * a.key_splits));
     hipLaunchKernelGGL(kern, grid, dim3(S::THREADS), 0, s, a);
     return check_launch("ti_gqa_prefill_paged");
   } else {
