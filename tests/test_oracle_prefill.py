@@ -189,3 +189,10 @@ def test_auto_schedule_from_host_bounds():
     assert not _choose_per_unit(2, 32, 4096, None, 512, True, 24, 4, 256, None)
     assert not _choose_per_unit(2, 32, 4096, 512, 512, False, 24, 4, 256, None)
     assert not per_unit(2, 1 << 21, None, 1024) and not per_unit(2, 1 << 21, 1024, 1024, causal=False)
+
+    # Ragged batches: a grid of the longest chunk's blocks for every sequence, most of them empty.
+    def ragged(longest, short, heads=(24, 4, 256)):
+        return _choose_per_unit(short + 1, longest + short, longest, 1020, 1024, True, *heads, None)
+    assert ragged(700, 63) and ragged(300, 511) and not ragged(1000, 511)
+    assert ragged(700, 255, (32, 8, 128)) and not ragged(1000, 511, (32, 8, 128))
+    assert _choose_per_unit(4000, 4000 * 300, 300, 900, 1024, True, 24, 4, 256, None)  # many, none empty

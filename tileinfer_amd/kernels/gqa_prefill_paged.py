@@ -88,6 +88,12 @@ def _per_unit_wins(q_len: int, kv_len: int, causal: bool, h_kv: int, group: int,
 # 40 of 300 over 600 331 / 319 (the one shape measured where the rule loses). One KV head of 256 and
 # 8 of 128 cross between 1,000 and 1,500 tokens too.
 _SHORT_CONTEXT = 1024
+# The grid of one workgroup per unit has the longest chunk's row blocks for every sequence; those past a
+# sequence's rows cost ~5 ns each, hidden while other units run. One chunk among many of one token, launched
+# workgroups, per unit / balanced, us: 24/4 heads of 256: 700 + 63 8,448 63 / 76, 300 + 511 30,720
+# 261 / 277, 700 + 255 33,792 173 / 167, 1,000 + 511 96,256 334 / 304; 32/8 of 128: 700 + 255 22,528
+# 229 / 224, 1,000 + 511 65,536 443 / 410. More empty ones than this are not launched.
+_EMPTY_BLOCKS = 32768
 
 
 def _choose_per_unit(batch: int, total_q: int, max_q: int, max_k: int | None, bound: int,
@@ -100,11 +106,15 @@ def _choose_per_unit(batch: int, total_q: int, max_q: int, max_k: int | None, bo
     loose = max_q > total_q or max_q * (h_q // h_kv) > 65535 * 128
     if causal and max_k is None and bound <= max_q and not loose:
         return True  # the table holds no more than the chunks
+    rows = 128 if d == 256 else 256           # rows of a workgroup (the kernel's launch shape)
     if batch != 1:
-        return not loose and (bound if max_k is None else min(max_k, bound)) <= _SHORT_CONTEXT
+        if loose or (bound if max_k is None else min(max_k, bound)) > _SHORT_CONTEXT:
+            return False
+        group = h_q // h_kv
+        empty = batch * -(-max_q * group // rows) - (-(-total_q * group // rows) + batch)
+        return h_kv * empty <= _EMPTY_BLOCKS
     if max_k is None:
         return False
-    rows = 128 if d == 256 else 256           # rows of a workgroup (the kernel's launch shape)
     wgs = torch.cuda.get_device_properties(dev).multi_processor_count
     return _per_unit_wins(int(total_q), int(max_k), bool(causal), h_kv, h_q // h_kv, rows, wgs)
 
