@@ -49,6 +49,23 @@ def test_declines_what_is_not_its_form():
             f(t)
 
 
+@pytest.mark.parametrize("case", ["missing", "not a module", "other torch"])
+def test_without_the_native_form(case, tmp_path, monkeypatch):
+    """Not built here, broken, or built for another torch: one warning, and every call is left to the
+    Python form; the library itself stays required."""
+    path = tmp_path / "_pycalls.so"
+    if case == "not a module":
+        path.write_bytes(b"not a shared object")
+    if case == "other torch":
+        path = _lib.CALLS_PATH
+        monkeypatch.setattr(torch, "__version__", "1.0.0")
+    monkeypatch.setattr(_lib, "CALLS_PATH", path)
+    monkeypatch.setattr(_lib, "_calls", None)
+    with pytest.warns(RuntimeWarning, match="host time"):
+        c = _lib.calls()
+    assert _lib.calls() is c and c.decode(*range(11)) is None and _lib.result(c.append(1)) is None
+
+
 def _strided(t):
     """t's values as every second row of a larger tensor (rows stay 16-byte aligned)."""
     out = torch.empty(t.shape[0], 2, *t.shape[1:], dtype=t.dtype, device=t.device)[:, 0]

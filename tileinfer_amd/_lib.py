@@ -2,14 +2,17 @@
 
 The library is loaded lazily on first use, after torch (torch's bundled HIP runtime has the same
 soname as ROCm's, so the kernels and torch share one runtime and torch's stream handles are valid
-here). There is no fallback: a missing library raises.
+here). There is no fallback: a missing library raises. (_pycalls.so beside it only saves host time; see
+:func:`calls`.)
 """
 from __future__ import annotations
 
 import ctypes
 import importlib.machinery
 import importlib.util
+import sys
 import threading
+import warnings
 from pathlib import Path
 
 import torch  # noqa: F401  (must be imported before the library: shared HIP runtime)
@@ -143,22 +146,43 @@ _BOUND = ("ti_kv_append", "ti_gqa_decode_plan", "ti_gqa_decode_paged", "ti_gqa_d
 _calls = None
 
 
+def versions() -> str:
+    """What _pycalls.so has to be built for: it reads torch's and Python's own structures."""
+    return f"torch {torch.__version__}, Python {sys.version_info[0]}.{sys.version_info[1]}"
+
+
+class _PythonForm:
+    """As the module, with every call left to the Python form of the entry point."""
+
+    def __getattr__(self, name):
+        return lambda *args: None
+
+
+def _load_calls(lib: ctypes.CDLL):
+    loader = importlib.machinery.ExtensionFileLoader("_pycalls", str(CALLS_PATH))
+    mod = importlib.util.module_from_spec(importlib.util.spec_from_loader("_pycalls", loader))
+    loader.exec_module(mod)
+    built_for = getattr(mod, "built_for", "other versions")
+    if built_for != versions():
+        raise ImportError(f"{CALLS_PATH} is built for {built_for}, this is {versions()}")
+    mod.bind(*(ctypes.cast(getattr(lib, n), ctypes.c_void_p).value for n in _BOUND))
+    return mod
+
+
 def calls():
-    """The native form of the Python entry points (csrc/pycalls.cpp), bound to the library."""
+    """The native form of the Python entry points (csrc/pycalls.cpp), bound to the library. Without it
+    (not built, or built for another torch or Python) the entry points run their Python form."""
     global _calls
     if _calls is None:
         lib = load()
         with _lock:
             if _calls is None:
-                if not CALLS_PATH.exists():
-                    raise RuntimeError(f"{CALLS_PATH} is missing: build it with "
-                                       "`python -m tileinfer_amd.build`")
-                loader = importlib.machinery.ExtensionFileLoader("_pycalls", str(CALLS_PATH))
-                mod = importlib.util.module_from_spec(
-                    importlib.util.spec_from_loader("_pycalls", loader))
-                loader.exec_module(mod)
-                mod.bind(*(ctypes.cast(getattr(lib, n), ctypes.c_void_p).value for n in _BOUND))
-                _calls = mod
+                try:
+                    _calls = _load_calls(lib)
+                except ImportError as e:
+                    warnings.warn(f"{e}: calls take 5 to 10 us more of host time until it is built here "
+                                  "with `python -m tileinfer_amd.build`", RuntimeWarning, stacklevel=3)
+                    _calls = _PythonForm()
     return _calls
 
 

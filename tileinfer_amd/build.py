@@ -62,20 +62,40 @@ def _compile(hipcc: str, src: Path, extra: list[str]) -> Path:
     return obj
 
 
+def _cxx() -> str | None:
+    """A host C++ compiler; ROCm's own where there is no other."""
+    rocm = Path(_hipcc()).resolve().parent.parent
+    for cand in (os.environ.get("CXX"), shutil.which("g++"), shutil.which("clang++"),
+                 str(rocm / "bin" / "amdclang++"), str(rocm / "llvm" / "bin" / "clang++")):
+        if cand and (os.path.exists(cand) or shutil.which(cand)):
+            return cand
+    return None
+
+
 def _build_calls() -> None:
-    """csrc/pycalls.cpp against torch's headers (host code only)."""
+    """csrc/pycalls.cpp against torch's and Python's headers (host code only). Where a host compiler or
+    the headers are missing it is left out, with a line that says so: the entry points then run their
+    Python form."""
     import torch
     from torch.utils import cpp_extension
 
-    cxx = os.environ.get("CXX") or shutil.which("g++") or shutil.which("clang++")
-    if cxx is None:
-        raise RuntimeError("no C++ compiler found for pycalls.cpp (set CXX)")
+    from ._lib import versions
+
+    cxx = _cxx()
+    includes = [*cpp_extension.include_paths(), sysconfig.get_paths()["include"]]
+    missing = [n for n in ("ATen/ATen.h", "Python.h")
+               if not any(os.path.exists(os.path.join(p, n)) for p in includes)]
+    missing += [] if cxx else ["a host C++ compiler"]
+    if missing:
+        CALLS_PATH.unlink(missing_ok=True)
+        print(f"{CALLS_PATH.name} left out ({', '.join(missing)} not found): calls take 5 to 10 us more "
+              "of host time", file=sys.stderr)
+        return
     tmp = CALLS_PATH.with_suffix(".so.tmp")
     lib_dir = Path(torch.__file__).resolve().parent / "lib"
     cmd = [cxx, "-O2", "-std=c++17", "-fPIC", "-shared", "-Wall",
-           f"-D_GLIBCXX_USE_CXX11_ABI={int(torch._C._GLIBCXX_USE_CXX11_ABI)}",
-           *(f"-isystem{p}" for p in cpp_extension.include_paths()),
-           f"-isystem{sysconfig.get_paths()['include']}", str(CSRC / "pycalls.cpp"), "-o", str(tmp),
+           f'-DTI_BUILT_FOR="{versions()}"', f"-D_GLIBCXX_USE_CXX11_ABI={int(torch._C._GLIBCXX_USE_CXX11_ABI)}",
+           *(f"-isystem{p}" for p in includes), str(CSRC / "pycalls.cpp"), "-o", str(tmp),
            f"-L{lib_dir}", "-ltorch_python", "-ltorch_cpu", "-lc10"]
     res = subprocess.run(cmd, capture_output=True, text=True)
     if res.returncode != 0:

@@ -385,4 +385,9 @@ PyModuleDef module = {PyModuleDef_HEAD_INIT, "_pycalls", nullptr, -1, methods,
 
 }  // namespace
 
-PyMODINIT_FUNC PyInit__pycalls(void) { return PyModule_Create(&module); }
+// built_for (given by the build): the versions whose structures this file was compiled against.
+PyMODINIT_FUNC PyInit__pycalls(void) {
+  PyObject* m = PyModule_Create(&module);
+  if (m && PyModule_AddStringConstant(m, "built_for", TI_BUILT_FOR) < 0) Py_CLEAR(m);
+  return m;
+}
