@@ -129,10 +129,11 @@ def test_append_bulk_65536(dev):
 
 
 @pytest.mark.parametrize("heads,d,around", [(4, 256, 1024), (4, 256, 16384), (1, 8, 1024), (1, 3, 1024)])
-@pytest.mark.parametrize("off", [-1, 0, 1, 7])
+@pytest.mark.parametrize("off", [-1, 0, 1, 2, 7])
 def test_append_at_the_lines_of_items_per_lane(heads, d, around, off, dev):
-    """One, two and four items per lane meet at 1,024 and 16,384 items per CU; counts off either line
-    leave lanes without an item, and skipped and out-of-range slots lie among them."""
+    """One, two and four items per lane meet at 1,024 and above 16,384 items per CU (with 256 CUs and 128
+    items a token two tokens more reach 16,385); counts off either line leave lanes without an item,
+    and skipped and out-of-range slots lie among them."""
     say(f"append lines {heads}x{d} {around} {off}")
     row = heads * d
     items = row // 8 if row % 8 == 0 else row  # 16-byte vectors, or single values
@@ -148,5 +149,23 @@ def test_append_at_the_lines_of_items_per_lane(heads, d, around, off, dev):
     live = (slots >= 0) & (slots < n + 9)
     for w, x in zip(want, (k, v)):
         w[slots[live].long()] = x.view(n, row)[live]
+    store_kvcache(k, v, kc, vc, slots)
+    assert torch.equal(bits(kc), bits(want[0])) and torch.equal(bits(vc), bits(want[1]))
+
+
+def test_append_above_one_trip_of_the_grid(dev):
+    """More than 32 * 1,024 items per CU: the workgroups loop, and their last trip is a partial one."""
+    cus = torch.cuda.get_device_properties(dev).multi_processor_count
+    n = 1024 * cus + 33  # 32 items a token
+    say(f"append, looping workgroups: {n} tokens")
+    g = torch.Generator(device=dev).manual_seed(6)
+    k, v = (torch.randn(n, 1, 256, generator=g, device=dev).to(torch.bfloat16) for _ in range(2))
+    slots = torch.randperm(n + 9, generator=g, device=dev)[:n].to(torch.int32)
+    slots[::97] = -1
+    kc, vc = (torch.full((n + 9, 256), 3.0, dtype=torch.bfloat16, device=dev) for _ in range(2))
+    want = [kc.clone(), vc.clone()]
+    live = slots >= 0
+    for w, x in zip(want, (k, v)):
+        w[slots[live].long()] = x.view(n, 256)[live]
     store_kvcache(k, v, kc, vc, slots)
     assert torch.equal(bits(kc), bits(want[0])) and torch.equal(bits(vc), bits(want[1]))

@@ -80,3 +80,31 @@ def test_values_outside_every_mask_stay_out(dev):
                                    schedule="balanced")
         keep = 400 if first == 470 else 352  # whole query blocks of 32 tokens before position 448
         assert torch.equal(bits(out[:keep]), bits(clean[:keep])), first
+
+
+@pytest.mark.parametrize("page", [16, 8, 4])
+def test_page_ids_outside_the_cache(page, dev):
+    """Ids outside the cache inside a context are absent keys, in cut units too (a few chunks over long
+    contexts: every unit is cut between workgroups): the rows are the attention over the other keys,
+    in 64 bits within the prefill tolerance."""
+    q_lens, kv_lens, hq, hkv, d = [20, 9], [3000, 1700], 4, 2, 256
+    step = prefill_step(q_lens, kv_lens, seed=54, hq=hq, hkv=hkv, page=page)
+    say(f"prefill pairs absent pages, page={page}")
+    nb = step.k_cache.shape[0]
+    for b, at, bad in ((0, 0, -1), (0, 1000, nb), (0, 1016, 10 ** 8), (0, 2999, -7), (1, 640, 2 ** 31 - 1)):
+        step.block_table[b, at // page] = bad
+    out = run(step, dev).cpu()
+    k, v = (c.reshape(-1, hkv, d).double() for c in (step.k_cache, step.v_cache))
+    at = 0
+    for b, (n, c) in enumerate(zip(q_lens, kv_lens)):
+        pos = torch.arange(c)
+        ids = step.block_table[b, pos // page].long()
+        pos = pos[(ids >= 0) & (ids < nb)]
+        rows = step.block_table[b, pos // page].long() * page + pos % page
+        assert len(pos) < c
+        seen = pos[None] <= c - n + torch.arange(n)[:, None]
+        for h in range(hq):
+            s = step.q[at:at + n, h].double() @ k[rows, h // (hq // hkv)].T / d ** 0.5
+            want = torch.softmax(s.masked_fill(~seen, float("-inf")), -1) @ v[rows, h // (hq // hkv)]
+            torch.testing.assert_close(out[at:at + n, h].double(), want, atol=ATOL, rtol=RTOL)
+        at += n

@@ -61,13 +61,17 @@ def test_tiny_pages_vs_oracle(page, variant, dev):
     assert_decode_close(out, ref)
 
 
+_HEADS = pytest.mark.parametrize("d,hq,hkv", [(256, 24, 4), (128, 32, 8)])
+
+
+@_HEADS
 @pytest.mark.parametrize("page", [8, 4, 2])
-def test_same_memory_as_page16_bitwise(page, dev):
+def test_same_memory_as_page16_bitwise(page, d, hq, hkv, dev):
     """A page-16 cache viewed as pages of `page` tokens (block i -> blocks 16/page * i + j) is the
     same tokens in the same 16-token tiles: the decode is bitwise the page-16 decode, under the
     balanced plan, a fixed split, and the forced cache policies; the fused append too."""
     ctx = [700, 4096, 33, 1, 2500, 9000, 16, 17]
-    st = _on(make_step(ctx, pool=1200, seed=51, width=600), dev)
+    st = _on(make_step(ctx, pool=1200, seed=51, width=600, hq=hq, hkv=hkv, d=d), dev)
     r = 16 // page
     nb = st.k_cache.shape[0]
     kv_small = [c.view(nb * r, page, *c.shape[2:]) for c in (st.k_cache, st.v_cache)]
@@ -93,31 +97,35 @@ def test_same_memory_as_page16_bitwise(page, dev):
     assert torch.equal(bits(k16), bits(st.k_cache)) and torch.equal(bits(v16), bits(st.v_cache))
 
 
+@_HEADS
 @pytest.mark.parametrize("page", [8, 4])
-def test_absent_pages_and_padding_rows(page, dev):
+def test_absent_pages_and_padding_rows(page, d, hq, hkv, dev):
     """An id outside the cache at a used position is an absent page (its tokens masked, never
-    read), also when it shares a 16-token tile with a present page; the runner's graph-padding
-    rows (context 1, all -1) decode to zeros."""
-    ctx = [100, 100, 40, 1]
-    st = make_step(ctx, pool=80, seed=52, page=page)
+    read), also when it shares a 16-token tile with a present page, the last, partial tile among
+    them; the runner's graph-padding rows (context 1, all -1) decode to zeros."""
+    ctx = [100, 100, 40, 1, 110, 110]
+    st = make_step(ctx, pool=160, seed=52, page=page, hq=hq, hkv=hkv, d=d)
     tbl = st.block_table.clone()
     tbl[0, 3] = 10**6               # one page of sequence 0
     tbl[1, 0] = -5                  # sequence 1's first page
     tbl[2, 1] = -1                  # sequence 2's second page
     tbl[3, :] = -1                  # padding row
-    say(f"small pages: absent pages, page={page}")
+    tbl[4, 109 // page] = 10**6     # the last, partial tile's last page
+    tbl[5, 96 // page] = 2**31 - 1  # and its first
+    say(f"small pages: absent pages, page={page} d={d}")
     out = gqa_decode_paged_fn(st.q.to(dev), st.k_cache.to(dev), st.v_cache.to(dev),
                               tbl.to(dev), st.seqlen.to(dev), page).cpu()
-    kf = st.k_cache.float().reshape(-1, 4, 256).double()
-    vf = st.v_cache.float().reshape(-1, 4, 256).double()
-    for b in range(3):
+    kf = st.k_cache.float().reshape(-1, hkv, d).double()
+    vf = st.v_cache.float().reshape(-1, hkv, d).double()
+    group = hq // hkv
+    for b in (0, 1, 2, 4, 5):
         pos = [p for p in range(ctx[b]) if 0 <= int(tbl[b, p // page]) < st.k_cache.shape[0]]
         assert len(pos) < ctx[b]
         rows = torch.tensor([int(tbl[b, p // page]) * page + p % page for p in pos])
         k, v = kf[rows], vf[rows]
-        for h in range(24):
-            w = torch.softmax(k[:, h // 6] @ st.q[b, h].double() / 16.0, 0)
-            torch.testing.assert_close(out[b, h].double(), w @ v[:, h // 6], atol=1e-2, rtol=1e-2)
+        for h in range(hq):
+            w = torch.softmax(k[:, h // group] @ st.q[b, h].double() / d ** 0.5, 0)
+            torch.testing.assert_close(out[b, h].double(), w @ v[:, h // group], atol=1e-2, rtol=1e-2)
     assert not bool(out[3].view(torch.int16).any())
 
 

@@ -19,18 +19,34 @@ class _Declines:
         return lambda *a: None
 
 
-def both(monkeypatch, call):
-    """call()'s tensors from either form (or the exception), and compares them."""
-    got = []
+class _Watched:
+    """As calls(), and notes in `taken` whether each call was taken (True) or declined (False)."""
+
+    def __init__(self, taken):
+        self.calls, self.taken = _lib.calls(), taken
+
+    def __getattr__(self, name):
+        def call(*a):
+            r = getattr(self.calls, name)(*a)
+            self.taken.append(r is not None)
+            return r
+        return call
+
+
+def both(monkeypatch, call, taken=None):
+    """call()'s tensors from either form (or the exception), and compares them. `taken`: whether the
+    native form has to have taken the call (True) or declined it (False)."""
+    got, seen = [], []
     for native in (True, False):
         with monkeypatch.context() as m:
-            if not native:
-                m.setattr(_lib, "calls", lambda: _Declines())
+            c = _Watched(seen) if native else _Declines()
+            m.setattr(_lib, "calls", lambda: c)
             try:
                 got.append(call())
             except Exception as e:  # noqa: BLE001 (compared by type)
                 got.append(type(e))
     a, b = got
+    assert taken is None or seen in ([[True]] if taken else [[], [False]]), seen
     if isinstance(a, type) or isinstance(b, type):
         assert a is b
         return a
@@ -97,6 +113,20 @@ def _expect(refused, form, wrong=False):
         assert refused is None
 
 
+def _taken(which, form, qknorm=False, append=False):
+    """Whether the native form takes the call: the plain form always; a parameter, but for the operand
+    whose type the entry point looks at; operands a stride apart where the kernels take strides (not
+    the gate, nor the vectors of one number per sequence or token); addresses off 16 bytes where they
+    take 4 or 2 (table, vectors, the input side)."""
+    if form == "parameter":
+        return which != ("k" if append else "q")
+    if form == "strided":
+        return which not in ("gate", "lens", "slots")
+    if form == "odd":
+        return which in ("table", "lens", "slots") or qknorm or append
+    return form == "plain"
+
+
 @pytest.mark.gpu
 @pytest.mark.parametrize("form", list(_FORMS))
 @pytest.mark.parametrize("which", ["q", "table", "lens", "gate", "key", "slots", "page"])
@@ -122,7 +152,9 @@ def test_decode(which, form, dev, monkeypatch):
         out = gqa_decode_paged_fn(f("q", d["q"]), k, v, f("table", d["block_table"]),
                                   f("lens", d["seqlen"]), page, **more)
         return out, k, v
-    refused = both(monkeypatch, call)
+    # (The gate's last two axes, one of them of size one, swapped are the same gate.)
+    refused = both(monkeypatch, call, which != "page" and (
+        _taken(which, form) or (which, form) == ("gate", "transposed")))
     _expect(refused, form, which == "page")
 
 
@@ -166,7 +198,7 @@ def test_prefill(schedule, which, form, dev, monkeypatch):
     # A shorter q is fewer tokens than cu_seqlens_q states, which only the device sees.
     if form == "short" and which == "q":
         pytest.skip("not a form to refuse on the host")
-    refused = both(monkeypatch, call)
+    refused = both(monkeypatch, call, _taken(which, form))
     _expect(refused, form)
 
 
@@ -193,10 +225,10 @@ def test_append_and_qknorm(which, form, dev, monkeypatch):
         kc, vc = torch.zeros(8, 512, dtype=q.dtype, device=dev), torch.zeros(8, 512, dtype=q.dtype, device=dev)
         store_kvcache(f("k", k), f("v", v), kc, vc, f("slots", slots))
         return kc, vc
-    refused = both(monkeypatch, qknorm)
+    refused = both(monkeypatch, qknorm, _taken(which, form, qknorm=True))
     if form == "wide" and which != "cos" or form == "short":
         assert refused is not None
-    both(monkeypatch, append)
+    both(monkeypatch, append, None if which in ("q", "cos") else _taken(which, form, append=True))
 
 
 @pytest.mark.gpu
