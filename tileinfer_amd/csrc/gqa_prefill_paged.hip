@@ -71,8 +71,12 @@ constexpr float kRescaleSlack = 8.f;  // exp2 units a row maximum may rise befor
 constexpr int kMinChunkTiles = 11;    // shortest run of key tiles of a balanced workgroup
 constexpr int kXcds = 8;              // MI355X: 8 XCDs of 32 CUs, one L2 each
 // A unit's start-up and epilogue (Q load, pipeline fill, output or partial store), priced in key
-// tiles. Measured: a causal 2,048-token first chunk (units of 1..64 tiles) takes 125 us at 2,
-// 109 at 4, 97.5 at 6, 96 at 9 and 100 at 14; long units (a 8,192-key continuation) do not move.
+// tiles. Whole balanced calls with the wave pairs at 4 / 6 / 9 / 14, us: a causal 2,048-token first
+// chunk (units of 1..64 tiles) 80 / 80 / 82 / 85, 24 chunks of 16 to 330 tokens over up to 2,000 cached
+// 188 / 184 / 170 / 166 and gated 237 / 227 / 202 / 190, 40 of 300 over 600 319 / 317 / 316 / 314; long
+// units (2,048 tokens over 8,192 keys) 319 / 320 / 321 / 325. head_dim 128, those 24 chunks:
+// 132 / 134 / 143 / 142. (kMinChunkTiles at 10, 11, 16: 2 chunks of 4 over 1,500 keys 34 / 34 / 37, the
+// others within 1 %.)
 constexpr int kUnitCost = 9;
 static_assert(kMinChunkTiles > kUnitCost, "every balanced run must reach a key tile");
 
@@ -1060,13 +1064,14 @@ __global__ __launch_bounds__(64 * W) void prefill_mfma_kernel(PrefillArgs a) {
 // layout, with the factors by which O has to be rescaled; one step later the output wave (waves
 // 4-7) adds V^T.P^T of that tile to the O it holds. A SIMD thus always has the MFMAs of P.V to run
 // beside the softmax, and every K or V operand read from LDS feeds C MFMAs: with O and Q in
-// different waves C = 3 column tiles fit the 256 registers of two waves per SIMD at head_dim 256,
-// where one wave holding both has room for one.
+// different waves C = 3 column tiles fit the 256 registers of two waves per SIMD at head_dim 256 (but
+// for a few values spilled outside the tile loops), where one wave holding both has room for one.
 //
-// K/V tiles of 32 keys go from the pages straight into LDS (buffer loads with the LDS
-// destination), K by the score waves two steps ahead of their use, V by the output waves as far
-// ahead, into rings of three stages each. One barrier per step publishes the tile of K, the tile
-// of V and the P^T of the step before. LDS rows are unpadded and swizzled (lds_swizzle) so that
+// K/V tiles of 32 keys go from the pages straight into LDS (buffer loads with the LDS destination).
+// The score waves describe the tiles to come (where their rows lie); the output waves issue the loads
+// of K and V two steps ahead of a tile's scores, K into a ring of three stages and V, which is read two
+// steps after K, into one of five. One barrier per step publishes the tiles that have landed and the
+// P^T of the step before. LDS rows are unpadded and swizzled (lds_swizzle) so that
 // the MFMA operand reads are free of bank conflicts.
 // P2: page_size is a power of two (page_shift >= 0); pages are then found with shifts (a runtime
 // division costs ~20 scalar instructions).
@@ -1075,12 +1080,14 @@ __global__ __launch_bounds__(64 * W) void prefill_mfma_kernel(PrefillArgs a) {
 // present in a tile are a bit mask (an absent page can share a sub-tile with a present one).
 //
 // What bounds it: on long runs the card's power limit. A continuation of 2,048 tokens over 8,192 keys
-// runs at 2.0 GHz (of 2.4) with the matrix cores busy 56 % of the cycles (2,726 a step, both waves
-// of a pair busy for 2,420 to 2,550 of them). Against the form before (12 waves of 16 rows, each
+// runs at 2.0 GHz (of 2.4; the other prefill launches at 2.1 to 2.2) with the matrix cores busy 51 %
+// of the launch's cycles and 56 % of the tile loop's (2,726 a step, both waves of a pair busy for 2,420
+// to 2,550 of them). Against the form before (12 waves of 16 rows, each
 // holding Q and O of its rows and reading every K and V operand for them alone: 2.7 times the LDS
-// reads), whole calls on one box: that continuation 363 -> 323 us, an 8,192-token prompt
-// 796 -> 712, six ragged chunks with context 257 -> 243, eight chunks of 16 over 8,000 keys
-// 75 -> 68; units of a few tiles are even (24 prompts of 17 to 700 tokens 130 -> 130).
+// reads), whole balanced calls on one box: that continuation 363 -> 323 us, an 8,192-token prompt
+// 796 -> 712 (where the caller asks for the balanced schedule: by default a first chunk runs per unit),
+// six ragged chunks with context 257 -> 243, eight chunks of 16 over 8,000 keys 75 -> 68; units of a few
+// tiles are even (24 prompts of 17 to 700 tokens 130 -> 130).
 // Why three stages of K and five of V: the loads of a tile are issued two steps before its scores
 // and land within one; V is read two steps after K. 192 rows take all 160 KiB so. Where in the step
 // the loads are issued makes no difference (within 2 %).

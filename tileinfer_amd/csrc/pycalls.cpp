@@ -1,8 +1,8 @@
 // The common form of the Python entry points in native code: argument checks, output and workspace
 // allocation and the library call, for calls whose operands are used as they are (plain CUDA tensors,
 // no copy to make, no option beyond those listed at each function). Anything else -- a wrong type,
-// shape, dtype, device, stride or alignment, a tensor subclass, an empty batch -- returns None, and
-// the Python function goes on with its own checks, which copy or raise.
+// shape, dtype, device, stride or alignment, a tensor subclass other than a parameter, an empty batch --
+// returns None, and the Python function goes on with its own checks, which copy or raise.
 //
 // Why: a call of this package is a few microseconds of GPU time at small sizes, and the Python
 // wrappers took 10 to 17 us of checks and argument conversion each, so that small calls were bound by

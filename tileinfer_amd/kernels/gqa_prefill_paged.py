@@ -25,9 +25,9 @@ work (units may be cut between workgroups and merged in fp32 afterwards, in a fi
 launches), which removes the partial last round of a continuation chunk and spreads a few long
 units over the whole GPU. ``schedule="auto"`` (default) picks per call from host-known sizes: the
 per-unit schedule when no sequence has cached context (``max_seqlen_k <= max_seqlen_q``: causal
-first chunks pack well heaviest-first) and for batches of contexts of at most 1,024 tokens, a greedy
-estimate of both for a single sequence, the balanced schedule otherwise. Without ``max_seqlen_k`` the
-block table's width bounds the contexts.
+first chunks pack well heaviest-first) and for batches of contexts of at most 1,024 tokens (unless they
+are so ragged that most of the grid would be empty), a greedy estimate of both for a single sequence,
+the balanced schedule otherwise. Without ``max_seqlen_k`` the block table's width bounds the contexts.
 """
 from __future__ import annotations
 
